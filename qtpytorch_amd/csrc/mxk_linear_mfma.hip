@@ -45,7 +45,7 @@
 // splits across workgroups (few rows) write partials that a second kernel
 // sums in split order.  Every reduction order is fixed, so results are
 // deterministic.
-#include "mxk_internal.h"
+#include "mxk_linear_mfma.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -54,18 +54,10 @@ namespace mxk {
 
 namespace {
 
-typedef _Float16 h8v __attribute__((ext_vector_type(8)));
-typedef _Float16 h2v __attribute__((ext_vector_type(2)));
-typedef float f4v __attribute__((ext_vector_type(4)));
-typedef uint32_t u4v __attribute__((ext_vector_type(4)));
-typedef uint32_t u2v __attribute__((ext_vector_type(2)));
-
 constexpr int LM_THREADS = 512;
 constexpr int LM_STAGE = 256;                  // rows of K per LDS stage
 constexpr int LM_FRAG = 1024;                  // one B fragment: 64 lanes x 8 f16
 constexpr int LM_STAGE_BYTES = 64 * LM_FRAG;   // 8 k steps x 8 column tiles
-constexpr uint32_t LM_OOB = 0x80000000u;       // past every buffer: loads return zeros
-constexpr size_t LM_WS_BASE = 65536;           // workspace bytes left to the decode kernels' counters
 
 // Slot of MFMA lane `lane` in the fragment of k step `ks`: a permutation of
 // the 16 slots of each 16-lane group, so that the fragment reads (16 lanes
@@ -76,101 +68,11 @@ __device__ __forceinline__ uint32_t lm_frag_off(int ks, int t, int lane) {
   return (uint32_t)((ks * 8 + t) * LM_FRAG + lm_slot(lane, ks) * 16);
 }
 
-// Two int4 codes at bits 0-3 and 16-19 of d (other bits ignored) as an f16
-// pair: 0x6400 | (c ^ 8) is the f16 1024 + (c + 8), exact, less 1032.
-__device__ __forceinline__ uint32_t lm_i4pair(uint32_t d) {
-  const uint32_t e = (d & 0x000F000Fu) ^ 0x64086408u;
-  const h2v r = __builtin_bit_cast(h2v, e) - h2v{(_Float16)1032.0f, (_Float16)1032.0f};
-  return __builtin_bit_cast(uint32_t, r);
-}
-// Two int8 codes at bits 0-7 and 16-23 of d (bits 8-15, 24-31 zero):
-// 0x6400 | (c ^ 0x80) is 1024 + (c + 128), less 1152.
-__device__ __forceinline__ uint32_t lm_i8pair(uint32_t d) {
-  const uint32_t e = d ^ 0x64806480u;
-  const h2v r = __builtin_bit_cast(h2v, e) - h2v{(_Float16)1152.0f, (_Float16)1152.0f};
-  return __builtin_bit_cast(uint32_t, r);
-}
-// Two int2 codes at bits 0-1 and 16-17 of d (other bits ignored):
-// 0x6400 | (c ^ 2) is 1024 + (c + 2), less 1026.
-__device__ __forceinline__ uint32_t lm_i2pair(uint32_t d) {
-  const uint32_t e = (d & 0x00030003u) ^ 0x64026402u;
-  const h2v r = __builtin_bit_cast(h2v, e) - h2v{(_Float16)1026.0f, (_Float16)1026.0f};
-  return __builtin_bit_cast(uint32_t, r);
-}
-// Two int1 codes at bits 0 and 16 of d (other bits ignored): code 0 is
-// +1 and code 1 is -1 (the reference's 1-bit grid), so the code is the f16
-// sign bit of 1.0.
-__device__ __forceinline__ uint32_t lm_i1pair(uint32_t d) { return ((d & 0x00010001u) << 15) | 0x3C003C00u; }
-// Weight formats: the code width in the low 4 bits, 16 for float grids
-enum : int { LM_I1 = 1, LM_I2 = 2, LM_I4 = 4, LM_I8 = 8, LM_F4 = 16 + 4, LM_F8 = 16 + 8 };
-__host__ __device__ constexpr int lm_bits(int fmt) { return fmt & 15; }
-// The factor the outputs take for B fragments that hold v * 2^-P instead of
-// the grid value v / vmax: RN(1/6) * 2^14, RN(1/480) * 2^8, or 1 for integer
-// codes.
-__host__ __device__ constexpr float lm_post(int fmt) {
-  return fmt == LM_F4 ? (1.0f / 6.0f) * 16384.0f : fmt == LM_F8 ? (1.0f / 480.0f) * 256.0f : 1.0f;
-}
-inline int lm_format(int kind, int bits) {
-  if (kind == MXK_KIND_INT) return bits == 1 ? LM_I1 : bits == 2 ? LM_I2 : bits == 4 ? LM_I4 : bits == 8 ? LM_I8 : 0;
-  if (kind == MXK_KIND_FLOAT) return bits == 4 ? LM_F4 : bits == 8 ? LM_F8 : 0;
-  return 0;
-}
-// Two codes of a format (layout of its width) as an f16 B-operand pair
-template <int FMT>
-__device__ __forceinline__ uint32_t lm_pair(uint32_t d) {
-  if constexpr (FMT == LM_I4) return lm_i4pair(d);
-  else if constexpr (FMT == LM_I8) return lm_i8pair(d);
-  else if constexpr (FMT == LM_I2) return lm_i2pair(d);
-  else if constexpr (FMT == LM_I1) return lm_i1pair(d);
-  else return fp_code_pair_f16<lm_bits(FMT)>(d);
-}
-
-// v_perm_b32 selector: byte a of s1 into byte 0, byte b of s0 into byte 2, zeros in bytes 1 and 3
-__host__ __device__ constexpr uint32_t lm_sel(int a, int b) {
-  return (uint32_t)a | 0x0C00u | ((uint32_t)(4 + b) << 16) | 0x0C000000u;
-}
-// the same bytes into bytes 1 and 3 (FP8 codes at the top of each half), zeros in bytes 0 and 2
-__host__ __device__ constexpr uint32_t lm_selh(int a, int b) {
-  return 0x0Cu | ((uint32_t)a << 8) | 0x0C0000u | ((uint32_t)(4 + b) << 24);
-}
-// the byte-pair selector a format's pair decoder takes
-template <int FMT>
-__host__ __device__ constexpr uint32_t lm_sel_f(int a, int b) {
-  return FMT == LM_F8 ? lm_selh(a, b) : lm_sel(a, b);
-}
-
-// p = x * s as f16 hi + lo for two elements: hi = RN16(x*s), lo =
-// RN16(x*s - hi), each one v_fma_mix (fp32 product, f16 result), so
-// |x*s - hi - lo| <= 2^-22 |x*s| (less for values whose lo is subnormal:
-// at most 2^-25 absolute).
-__device__ __forceinline__ void lm_split2(float x0, float s0, float x1, float s1, uint32_t& hi, uint32_t& lo) {
-  uint32_t h, l;
-  asm("v_fma_mixlo_f16 %0, %1, %2, 0 op_sel_hi:[0,0,0]" : "=v"(h) : "v"(x0), "v"(s0));
-  asm("v_fma_mixhi_f16 %0, %1, %2, 0 op_sel_hi:[0,0,0]" : "+v"(h) : "v"(x1), "v"(s1));
-  asm("v_fma_mixlo_f16 %0, %1, %2, -%3 op_sel_hi:[0,0,1]" : "=v"(l) : "v"(x0), "v"(s0), "v"(h));
-  asm("v_fma_mixhi_f16 %0, %1, %2, -%3 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "+v"(l) : "v"(x1), "v"(s1), "v"(h));
-  hi = h;
-  lo = l;
-}
-
-// s_barrier after this wave's LDS stores are done; global loads still in
-// flight (prefetches) stay in flight.
-__device__ __forceinline__ void lm_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
 // ---------------------------------------------------------------- [K][N] stage decode
 // Thread (r8 = tid / 16, c8 = tid % 16) decodes rows 8 r8 .. +7 and columns
 // 8 c8 .. +7 of the stage: for column tile t the 8 codes of column 8 c8 + t,
 // which are the B fragment of MFMA lane c8 + 16 (r8 % 4) in k step r8 / 4.
 // A wave's threads are k step w, lanes 0..63 in order.
-template <int BITS>
-struct KnCodes {
-  uint32_t w[BITS == 8 ? 16 : 8];
-};
-
 // `dead` is 0 or LM_OOB: every loader's byte offsets are or-ed with it, so
 // that a load the caller does not need still issues (the compiler's wait
 // counts then stay exact across loop iterations) and reads zeros.
@@ -195,34 +97,6 @@ __device__ __forceinline__ void kn_load(KnCodes<BITS>& c, __amdgpu_buffer_rsrc_t
       c.w[2 * i + 1] = v[1];
     }
   }
-}
-
-// the B fragment of column tile t (column 8 c8 + t) from the thread's block
-template <int FMT>
-__device__ __forceinline__ u4v kn_frag(const KnCodes<lm_bits(FMT)>& c, int t) {
-  constexpr int BITS = lm_bits(FMT);
-  u4v f;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    if constexpr (BITS == 1) {
-      // rows 2q and 2q+1 (8 bits each) 16 bits apart: column 8 c8 + t at bits t, 16 + t
-      const uint32_t d = c.w[2 * q] | (c.w[2 * q + 1] << 16);
-      f[q] = lm_pair<FMT>(d >> t);
-    } else if constexpr (BITS == 2) {
-      // rows 2q and 2q+1 (16 bits each) side by side: column 8 c8 + t at bits 2t, 2t + 1
-      const uint32_t d = c.w[2 * q] | (c.w[2 * q + 1] << 16);
-      f[q] = lm_pair<FMT>(d >> (2 * t));
-    } else if constexpr (BITS == 4) {
-      // byte t/2 of rows 2q and 2q+1: the low nibbles are column 8 c8 + t for even t
-      const uint32_t d = __builtin_amdgcn_perm(c.w[2 * q + 1], c.w[2 * q], lm_sel(t >> 1, t >> 1));
-      f[q] = lm_pair<FMT>((t & 1) ? d >> 4 : d);
-    } else {
-      const int h = t >> 2, u = t & 3;
-      f[q] = lm_pair<FMT>(
-          __builtin_amdgcn_perm(c.w[2 * (2 * q + 1) + h], c.w[2 * (2 * q) + h], lm_sel_f<FMT>(u, u)));
-    }
-  }
-  return f;
 }
 
 template <int FMT>
@@ -429,18 +303,6 @@ __device__ __forceinline__ void nk_store_tiled(const NkCodes<4>& c, uint8_t* sB,
     }
   }
 }
-
-// x' (and its f16 hi / lo) in HBM as tiles of 16 rows x 8 columns of K,
-// tile (m / 16, k / 8) at element ((m / 16) * Kp/8 + k / 8) * 128 and
-// element (m % 16) * 8 + k % 8 inside it, so that the 64 lanes of an A
-// operand load (rows j of a row tile, columns 8 g .. 8 g + 7 of a k step)
-// read one contiguous 2 KiB (fp32) or 1 KiB (f16): with x' row-major the 16
-// rows of one load are Kp elements apart and land on one memory channel.
-__host__ __device__ __forceinline__ int64_t lm_xoff(int64_t m, int64_t k, int64_t Kp) {
-  return ((m >> 4) * (Kp >> 3) + (k >> 3)) * 128 + (m & 15) * 8 + (k & 7);
-}
-// rows of x' the tiled layout holds (whole row tiles)
-__host__ __device__ __forceinline__ int64_t lm_rows16(int64_t M) { return (M + 15) & ~(int64_t)15; }
 
 // ---------------------------------------------------------------- the MFMA kernel
 // A-operand registers of one k step: [K][N] x' (2 row tiles x 8 fp32) and
@@ -651,7 +513,7 @@ __global__ __launch_bounds__(LM_THREADS, 1) void k_linear_mfma(
         h8v ahi[2], alo[2];
         build(ar[p], ahi, alo);
         load_step(ar[p], gs + 2);
-        __builtin_amdgcn_sched_barrier(0);
+        lm_settle();
         mfmas(ahi, alo, bt, 0, 8);
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -696,7 +558,7 @@ __global__ __launch_bounds__(LM_THREADS, 1) void k_linear_mfma(
         } else {
           load_step(ar[p], gs + 2);
         }
-        __builtin_amdgcn_sched_barrier(0);
+        lm_settle();
         mfmas(ahi, alo, bt, 0, BT);
         if constexpr (NK) {
 #pragma unroll
@@ -792,133 +654,6 @@ __global__ __launch_bounds__(256) void k_linear_mfma_reduce(const float* __restr
   *reinterpret_cast<f4v*>(out + 4 * q) = y;
 }
 
-// ---------------------------------------------------------------- prepasses
-// Row m of x: ex[m] such that its largest |x| times 2^ex lies in [1, 2)
-// (0 for a zero row), and x * 2^ex zero-padded to Kp columns, as fp32
-// (SPLIT false) or as f16 hi + lo (SPLIT true: hi = RN16(v), lo = RN16(v - hi),
-// v - hi exact in fp32).  VEC: 16-byte rows (K * sizeof(T) % 16 == 0, x
-// 16-byte aligned); rows of up to 2048 16-byte chunks stay in registers
-// between the maximum and the scaled copy, longer ones are read twice.
-template <typename T, bool SPLIT>
-__device__ __forceinline__ void lm_put(float* __restrict__ xs, _Float16* __restrict__ xh, _Float16* __restrict__ xl,
-                                       int64_t at, float v) {
-  if constexpr (SPLIT) {
-    const _Float16 h = (_Float16)v;
-    xh[at] = h;
-    xl[at] = (_Float16)(v - (float)h);
-  } else {
-    xs[at] = v;
-  }
-}
-
-//
-// Workgroups M .. M + NB - 1 (the [K][N] product) find es[nb] instead: the
-// power of two that puts the largest |scale| of column block nb (row nb of
-// the block-major scales sT [NB][K]) in [2^13, 2^14), 0 for a zero or
-// non-finite maximum.  It depends on the weight alone; computed here, it is
-// ready before the main kernel starts.
-template <typename T, bool SPLIT, bool VEC>
-__global__ __launch_bounds__(256) void k_linear_mfma_prep_rows(const T* __restrict__ x, int64_t M, int64_t K,
-                                                               int64_t Kp, float* __restrict__ xs,
-                                                               _Float16* __restrict__ xh, _Float16* __restrict__ xl,
-                                                               int* __restrict__ ex, const float* __restrict__ sT,
-                                                               int* __restrict__ es) {
-  constexpr int E = 16 / (int)sizeof(T), NCH = 8;
-  __shared__ float red[4];
-  const int tid = threadIdx.x;
-  if ((int64_t)blockIdx.x >= M) {
-    const int64_t nb = (int64_t)blockIdx.x - M;
-    const float* s = sT + nb * K;
-    float mx = 0.0f;
-    int64_t k = tid;
-    for (; k + 7 * 256 < K; k += 8 * 256) {
-      float v[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = s[k + 256 * u];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) mx = fmaxf(mx, __builtin_fabsf(v[u]));
-    }
-    for (; k < K; k += 256) mx = fmaxf(mx, __builtin_fabsf(s[k]));
-    mx = group_max<64>(mx);
-    if ((tid & 63) == 0) red[tid >> 6] = mx;
-    __syncthreads();
-    if (tid == 0) {
-      mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-      const int be = (int)((__float_as_uint(mx) >> 23) & 0xFFu);
-      es[nb] = (be == 0xFF || mx == 0.0f) ? 0 : 140 - (be == 0 ? 1 : be);
-    }
-    return;
-  }
-  const int64_t m = blockIdx.x;
-  const T* row = x + m * K;
-  const int64_t nch = K / E;
-  const bool cached = VEC && nch <= (int64_t)NCH * 256;
-  u4v c[NCH];
-  auto elems = [&](const u4v& w, float (&v)[E]) {
-    const T* t = reinterpret_cast<const T*>(&w);
-#pragma unroll
-    for (int e = 0; e < E; ++e) v[e] = ElemT<T>::cvt(t[e]);
-  };
-  float mx = 0.0f;
-  if (cached) {
-#pragma unroll
-    for (int q = 0; q < NCH; ++q) {
-      const int64_t ch = tid + 256 * q;
-      c[q] = ch < nch ? *reinterpret_cast<const u4v*>(row + ch * E) : u4v{0u, 0u, 0u, 0u};
-    }
-#pragma unroll
-    for (int q = 0; q < NCH; ++q) {
-      float v[E];
-      elems(c[q], v);
-#pragma unroll
-      for (int e = 0; e < E; ++e) mx = fmaxf(mx, __builtin_fabsf(v[e]));
-    }
-  } else {
-    for (int64_t k = tid; k < K; k += 256) mx = fmaxf(mx, __builtin_fabsf(ElemT<T>::cvt(row[k])));
-  }
-  mx = group_max<64>(mx);
-  if ((tid & 63) == 0) red[tid >> 6] = mx;
-  __syncthreads();
-  mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-  const int be = (int)((__float_as_uint(mx) >> 23) & 0xFFu);
-  const int e = (be == 0xFF || mx == 0.0f) ? 0 : 127 - (be == 0 ? 1 : be);
-  if (tid == 0) ex[m] = e;
-  if (cached) {
-#pragma unroll
-    for (int q = 0; q < NCH; ++q) {
-      const int64_t ch = tid + 256 * q;
-      if (ch >= nch) break;
-      float v[E];
-      elems(c[q], v);
-#pragma unroll
-      for (int u = 0; u < E; ++u) v[u] = __builtin_ldexpf(v[u], e);
-      const int64_t at = lm_xoff(m, ch * E, Kp);  // E <= 8 values within one 8-column group
-      if constexpr (SPLIT) {
-        _Float16 h[E], l[E];
-#pragma unroll
-        for (int u = 0; u < E; ++u) {
-          h[u] = (_Float16)v[u];
-          l[u] = (_Float16)(v[u] - (float)h[u]);
-        }
-        if constexpr (E == 4) {
-          *reinterpret_cast<u2v*>(xh + at) = __builtin_bit_cast(u2v, h);
-          *reinterpret_cast<u2v*>(xl + at) = __builtin_bit_cast(u2v, l);
-        } else {
-          *reinterpret_cast<u4v*>(xh + at) = __builtin_bit_cast(u4v, h);
-          *reinterpret_cast<u4v*>(xl + at) = __builtin_bit_cast(u4v, l);
-        }
-      } else {
-#pragma unroll
-        for (int u = 0; u < E; u += 4) *reinterpret_cast<f4v*>(xs + at + u) = f4v{v[u], v[u + 1], v[u + 2], v[u + 3]};
-      }
-    }
-    for (int64_t k = K + tid; k < Kp; k += 256) lm_put<T, SPLIT>(xs, xh, xl, lm_xoff(m, k, Kp), 0.0f);
-  } else {
-    for (int64_t k = tid; k < Kp; k += 256)
-      lm_put<T, SPLIT>(xs, xh, xl, lm_xoff(m, k, Kp), k < K ? __builtin_ldexpf(ElemT<T>::cvt(row[k]), e) : 0.0f);
-  }
-}
-
 // Block-major copy sT[nb][k] = s[k][nb] of a [K][N] weight's scales (when
 // the caller has none)
 __global__ __launch_bounds__(256) void k_linear_mfma_scales_t(const float* __restrict__ s, int64_t K, int64_t NB,
@@ -935,8 +670,6 @@ struct LmPlan {
   int64_t Kp = 0;
   size_t off_ex = 0, off_es = 0, off_x = 0, off_s = 0, off_p = 0, bytes = 0;
 };
-
-inline size_t lm_round(size_t v) { return (v + 255) & ~(size_t)255; }
 
 // Largest row tile (WM) per kernel: the [N][K] kernel holds a second set of
 // accumulators (the block sums), so its wider tiles would spill registers.
@@ -1007,28 +740,6 @@ void lm_launch_w(const LmPlan& p, hipStream_t st, const float* xs, const _Float1
     case 2: lm_launch_t<FMT, 2, NK, TILED>(p, st, xs, xh, xl, sc, sc_kbm, ex, es, w, M, K, N, bias, out, part); break;
     default: lm_launch_t<FMT, 1, NK, TILED>(p, st, xs, xh, xl, sc, sc_kbm, ex, es, w, M, K, N, bias, out, part); break;
   }
-}
-
-// rows of x (and, with sT, the NB column-block exponents of a [K][N] weight)
-template <typename T, bool SPLIT>
-void lm_prep_rows_t(const T* x, int64_t M, int64_t K, int64_t Kp, float* xs, _Float16* xh, _Float16* xl, int* ex,
-                    const float* sT, int64_t NB, int* es, hipStream_t st) {
-  const dim3 grid((unsigned)(M + (sT ? NB : 0)));
-  if (aligned16(x) && (K * (int64_t)sizeof(T)) % 16 == 0)
-    hipLaunchKernelGGL((k_linear_mfma_prep_rows<T, SPLIT, true>), grid, dim3(256), 0, st, x, M, K, Kp, xs, xh, xl, ex,
-                       sT, es);
-  else
-    hipLaunchKernelGGL((k_linear_mfma_prep_rows<T, SPLIT, false>), grid, dim3(256), 0, st, x, M, K, Kp, xs, xh, xl,
-                       ex, sT, es);
-}
-
-template <bool SPLIT>
-void lm_prep_rows(const void* x, int x_type, int64_t M, int64_t K, int64_t Kp, float* xs, _Float16* xh, _Float16* xl,
-                  int* ex, const float* sT, int64_t NB, int* es, hipStream_t st) {
-  if (x_type == MXK_IN_F32) lm_prep_rows_t<float, SPLIT>((const float*)x, M, K, Kp, xs, xh, xl, ex, sT, NB, es, st);
-  else if (x_type == MXK_IN_F16)
-    lm_prep_rows_t<__half, SPLIT>((const __half*)x, M, K, Kp, xs, xh, xl, ex, sT, NB, es, st);
-  else lm_prep_rows_t<hip_bfloat16, SPLIT>((const hip_bfloat16*)x, M, K, Kp, xs, xh, xl, ex, sT, NB, es, st);
 }
 
 bool lm_common_ok(int64_t M, int64_t K, int64_t N, int kind, int bits, int block, int x_type, const float* out) {
