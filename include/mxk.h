@@ -36,7 +36,7 @@
 extern "C" {
 #endif
 
-#define MXK_ABI_VERSION 10
+#define MXK_ABI_VERSION 11
 
 typedef enum {
   MXK_OK = 0,
@@ -165,6 +165,16 @@ int mxk_qgemm(const void* a_packed, const float* a_scales, int64_t a_nscales, co
  * scales when w_scales_t is NULL and any K-split partials, all after the
  * counter prefix, which it leaves alone. */
 size_t mxk_linear_workspace(int64_t M, int64_t K, int64_t N, int bits, int block);
+
+/* Workspace bytes with which mxk_linear_wq and mxk_linear_wq_nt run the
+ * matrix-core kernel for weights that neither of their workspace queries
+ * counts: N (mxk_linear_wq) or K (mxk_linear_wq_nt) no multiple of 128, or
+ * blocks other than 128 (at least 8), 1-, 2-, 4- and 8-bit codes on 4-byte
+ * aligned buffers of whole 4-byte words.  0 for shapes the kernel does not
+ * take.  The workspace is optional: with a smaller one (or none) the scalar
+ * kernel runs.  Its first 64 KiB are left alone; the rest need not be
+ * cleared.  Calls sharing a workspace must not overlap. */
+size_t mxk_linear_ragged_workspace(int64_t M, int64_t K, int64_t N, int bits, int block);
 
 /* Block-major copy of a weight's scales for the decode path: w_scales_t[b][k]
  * = w_scales[k * (N/128) + b], i.e. [N/128][K] from the [K][N/128] layout

@@ -21,7 +21,7 @@ MXK_IN_F32, MXK_IN_F16, MXK_IN_BF16 = 0, 1, 2
 MXK_KIND_INT, MXK_KIND_FLOAT = 0, 1
 MXK_VAR_BASE, MXK_VAR_HADAMARD, MXK_VAR_VECTOR = 0, 1, 2
 MXK_DYN_PER_TOKEN, MXK_DYN_PER_CHANNEL, MXK_DYN_PER_TENSOR = 0, 1, 2
-ABI_VERSION = 10
+ABI_VERSION = 11
 
 _lock = threading.Lock()
 _lib = None
@@ -48,6 +48,7 @@ SIGNATURES = {
     "mxk_qgemm": (c_int, [c_vp, c_vp, c_i64, c_vp, c_vp, c_i64, c_i64, c_i64, c_i64, c_int, c_int, c_int,
                           c_vp, c_i64, c_vp, c_vp, c_vp, c_vp, c_sz, c_vp]),
     "mxk_linear_workspace": (c_sz, [c_i64, c_i64, c_i64, c_int, c_int]),
+    "mxk_linear_ragged_workspace": (c_sz, [c_i64, c_i64, c_i64, c_int, c_int]),
     "mxk_linear_wq": (c_int, [c_vp, c_int, c_i64, c_i64, c_vp, c_vp, c_vp, c_i64, c_int, c_int, c_int, c_vp,
                               c_vp, c_vp, c_sz, c_vp]),
     "mxk_linear_prepack_scales": (c_int, [c_vp, c_i64, c_i64, c_int, c_vp, c_vp]),

@@ -692,6 +692,18 @@ int linear_mfma_nk_tiled(const void* x, int x_type, int64_t M, int64_t K, const 
                          const float* w_scales_t, int64_t N, const float* bias, float* out, void* workspace,
                          size_t workspace_nbytes, hipStream_t st);
 
+// MFMA weight-only linear over weights whose blocks do not line up with
+// 128-column tiles (mxk_linear_ragged.hip): bytes of workspace (0 for shapes it
+// does not take), and the products, which return MXK_EUNSUPPORTED with nothing
+// launched for shapes, alignments or workspaces they do not take.
+size_t linear_ragged_workspace(int64_t M, int64_t K, int64_t N, int bits, int64_t block);
+int linear_ragged_kn(const void* x, int x_type, int64_t M, int64_t K, const void* w, int64_t w_nbytes,
+                     const float* scales, int64_t nscales, int64_t N, int kind, int bits, int block,
+                     const float* bias, float* out, void* workspace, size_t workspace_nbytes, hipStream_t st);
+int linear_ragged_nk(const void* x, int x_type, int64_t M, int64_t K, const void* w, int64_t w_nbytes,
+                     const float* scales, int64_t nscales, int64_t N, int kind, int bits, int block,
+                     const float* bias, float* out, void* workspace, size_t workspace_nbytes, hipStream_t st);
+
 // 'v'-rule requantization of a float32 buffer (GEMM outputs), mxtorch.py:1372-1385.
 int requant_vec_f32(const float* x, int64_t n, int bits, int block, void* packed, int64_t packed_nbytes,
                     float* scales, int64_t n_store, void* ws, size_t ws_bytes, hipStream_t st);

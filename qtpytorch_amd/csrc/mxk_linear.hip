@@ -1949,6 +1949,10 @@ size_t mxk_linear_workspace(int64_t M, int64_t K, int64_t N, int bits, int block
   return std::max(std::max(a, b), c);
 }
 
+size_t mxk_linear_ragged_workspace(int64_t M, int64_t K, int64_t N, int bits, int block) {
+  return linear_ragged_workspace(M, K, N, bits, block);
+}
+
 int mxk_linear_prepack_weight(const void* w_packed, int64_t K, int64_t N, int bits, int block, void* w_tiled,
                               void* stream) {
   if (!w_packed || !w_tiled) return fail(MXK_EINVAL, "linear_prepack_weight: null pointer");
@@ -2066,6 +2070,11 @@ static int linear_wq_impl(const void* x, int x_type, int64_t M, int64_t K, const
   }
   const int64_t nb = ceil_div(K * N, block);
   const int64_t pbytes = mxk_packed_nbytes(bits, nb * block);
+  {
+    const int rc = linear_ragged_kn(x, x_type, M, K, w_packed, pbytes, w_scales, nb, N, kind, bits, block, bias, out,
+                                    workspace, workspace_nbytes, st);
+    if (rc != MXK_EUNSUPPORTED) return rc;
+  }
   const uint8_t* pk = reinterpret_cast<const uint8_t*>(w_packed);
   if (x_type == MXK_IN_F32)
     return linear_t<false, float>((const float*)x, M, K, N, pk, pbytes, w_scales, kind, bits, block, bias, out, st);
@@ -2148,6 +2157,11 @@ int mxk_linear_wq_nt(const void* x, int x_type, int64_t M, int64_t K, const void
   {
     const int rc = linear_mfma_nk(x, x_type, M, K, w_packed, w_scales, w_scales_t, N, kind, bits, block, bias, out,
                                   workspace, workspace_nbytes, st);
+    if (rc != MXK_EUNSUPPORTED) return rc;
+  }
+  {
+    const int rc = linear_ragged_nk(x, x_type, M, K, w_packed, w_nbytes, w_scales, w_nscales, N, kind, bits, block,
+                                    bias, out, workspace, workspace_nbytes, st);
     if (rc != MXK_EUNSUPPORTED) return rc;
   }
   if (x_type == MXK_IN_F32)

@@ -448,7 +448,8 @@ def linear_wq(x: Tensor, w_packed: Optional[Tensor], w_scales: Tensor, dt, in_fe
     if b is not None and b.data_ptr() % 16:
         b = b.clone()
     lib = L.lib()
-    ws_bytes = lib.mxk_linear_workspace(M, K, N, dt.bits, block)
+    ws_bytes = (lib.mxk_linear_workspace(M, K, N, dt.bits, block)
+                or lib.mxk_linear_ragged_workspace(M, K, N, dt.bits, block))
     stream = L.stream_of(xc)
     ws = _zeroed_workspace(ws_bytes, dev, stream)
     with L.on_device(dev):
@@ -650,7 +651,8 @@ def linear_wq_nt(x: Tensor, w_packed: Optional[Tensor], w_scales: Tensor, dt, ou
             raise L.MXKError("linear_wq_nt: w_tiled must be prepack_weight_nt() of this weight (uint8, "
                              "contiguous, same device)")
     lib = L.lib()
-    ws_bytes = lib.mxk_linear_nt_workspace(M, K, N, dt.bits, block)
+    ws_bytes = (lib.mxk_linear_nt_workspace(M, K, N, dt.bits, block)
+                or lib.mxk_linear_ragged_workspace(M, K, N, dt.bits, block))
     stream = L.stream_of(xc)
     wk = _zeroed_workspace(ws_bytes, dev, stream)
     with L.on_device(dev):

@@ -1,0 +1,143 @@
+"""The weight-only linear over weights whose blocks do not line up with
+128-column tiles: out_features (mx_linear) or in_features ([out, in] weights)
+no multiple of 128, or blocks other than 128.
+
+Checked against x.double() @ dequant(W).double() with the oracle's dequantized
+weight.  The kernel carries x and c * s as f16 pairs hi + lo and leaves out lo
+* lo: each term is off by at most 3 * 2^-22 of itself, the fp32 sums add at
+most one rounding of 2^-24 per 32 terms and partial, and a value far below
+its row's (column tile's) largest keeps 2^-25 of that largest."""
+import pytest
+import torch
+
+from oracle import mx_oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+FMTS = ["int1d", "int2d", "int4d", "int8d", "float4d", "float8d"]
+
+
+@pytest.fixture(scope="module")
+def qa():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import qtpytorch_amd
+    return qtpytorch_amd
+
+
+def _case(M, K, N, dt, block, nt, src, seed=0):
+    g = torch.Generator().manual_seed(1000 * M + 10 * K + N + seed)
+    x = torch.randn(M, K, generator=g).to(src)
+    w = 0.02 * torch.randn(*((N, K) if nt else (K, N)), generator=g)
+    w[torch.rand(w.shape, generator=g) < 1e-2] *= 20
+    packed, scales, n = orc.quantize(w, dt, block)
+    return x, packed, scales, orc.dequant(packed, scales, dt, n, block).reshape(w.shape)
+
+
+def _run(qa, x, packed, scales, dt, K, N, block, nt, bias=None):
+    d = "cuda:0"
+    fn = qa.ops.linear_wq_nt if nt else qa.ops.linear_wq
+    sizes = (N, K) if nt else (K, N)
+    return fn(x.to(d), packed.to(d), scales.to(d), dt, *sizes, block, bias=None if bias is None else bias.to(d)).cpu()
+
+
+def _check(y, x, wd, nt, bias=None):
+    xd, w = x.double(), (wd.t() if nt else wd).double()
+    ref = xd @ w + (0 if bias is None else bias.double())
+    K = x.shape[1]
+    terms = xd.abs() @ w.abs()
+    floor = xd.abs().amax(1, keepdim=True) * w.abs().sum(0) * 2.0 ** -24
+    tol = (3 * 2.0 ** -22 + (K / 32 + 16) * 2.0 ** -24) * terms + floor + 2.0 ** -23 * ref.abs() + 1e-37
+    err = (y.double() - ref).abs()
+    assert bool((err <= tol).all()), f"worst {float((err / tol).max()):.3g} x the bound"
+
+
+SHAPES = [  # rows: edges of the 16-, 32- and 64-row tiles and of the waves along rows; columns around a tile; K around a step
+    (1, 33, 1), (16, 64, 127), (17, 95, 129), (32, 200, 1000), (33, 31, 257), (64, 1000, 130), (65, 129, 259),
+    (129, 257, 300), (300, 96, 391), (5, 4096, 203), (16, 1, 7), (3, 2049, 1001),
+]
+
+
+@pytest.mark.parametrize("nt", [False, True], ids=["kn", "nk"])
+@pytest.mark.parametrize("dt", FMTS)
+def test_shapes(qa, dt, nt):
+    for i, (M, K, N) in enumerate(SHAPES):
+        if nt:
+            K, N = N, K
+        src = (torch.float32, torch.bfloat16, torch.float16)[i % 3]
+        x, p, s, wd = _case(M, K, N, dt, 128, nt, src)
+        bias = torch.randn(N) if i % 2 else None
+        _check(_run(qa, x, p, s, dt, K, N, 128, nt, bias), x, wd, nt, bias)
+
+
+@pytest.mark.parametrize("nt", [False, True], ids=["kn", "nk"])
+@pytest.mark.parametrize("block", [8, 20, 64, 96, 200, 1000])
+def test_blocks(qa, block, nt):
+    for dt in ("int4d", "int8d", "float8d"):
+        for M, K, N in ((4, 160, 256), (70, 133, 77)):
+            x, p, s, wd = _case(M, K, N, dt, block, nt, torch.float32)
+            _check(_run(qa, x, p, s, dt, K, N, block, nt), x, wd, nt)
+
+
+@pytest.mark.parametrize("nt", [False, True], ids=["kn", "nk"])
+def test_magnitudes(qa, nt):
+    """Rows of x and blocks of W of very different magnitudes, and a zero row."""
+    M, K, N = 40, 513, 321
+    x, _, _, _ = _case(M, K, N, "int8d", 128, nt, torch.float32)
+    x *= 10.0 ** torch.linspace(-7, 7, M)[:, None]
+    x[3] = 0
+    for e in (1e-6, 1e6):
+        w = e * torch.randn(*((N, K) if nt else (K, N)), generator=torch.Generator().manual_seed(5))
+        p, s, n = orc.quantize(w, "int8d", 128)
+        wd = orc.dequant(p, s, "int8d", n, 128).reshape(w.shape)
+        y = _run(qa, x, p, s, "int8d", K, N, 128, nt)
+        _check(y, x, wd, nt)
+        assert not y[3].any()
+
+
+@pytest.mark.parametrize("nt", [False, True], ids=["kn", "nk"])
+@pytest.mark.parametrize("M", [3, 70])
+def test_non_finite(qa, nt, M):
+    """Infinities and NaN in x and in the scales come out where an fp32 product has them."""
+    K, N = 300, 203
+    x, p, s, wd = _case(M, K, N, "int8d", 128, nt, torch.float32)
+    x[0, 7] = float("inf")
+    x[1, 9] = float("nan")
+    s[5] = float("inf")
+    wd = orc.dequant(p, s, "int8d", K * N, 128).reshape(wd.shape)
+    y = _run(qa, x, p, s, "int8d", K, N, 128, nt)
+    ref = x.double() @ (wd.t() if nt else wd).double()
+    assert torch.equal(y.isnan(), ref.isnan()) and torch.equal(y.isinf(), ref.isinf())
+    assert torch.equal(y[y.isinf()].sign().double(), ref[ref.isinf()].sign())
+    fin = ref.isfinite()
+    assert float(((y.double() - ref)[fin]).abs().max()) <= 1e-3 * float(ref[fin].abs().max())
+
+
+def test_module_and_gradient(qa):
+    """mx_linear with an odd width: forward, input gradient and a captured replay."""
+    g = torch.Generator().manual_seed(3)
+    lin = torch.nn.Linear(160, 203, bias=False)
+    with torch.no_grad():
+        lin.weight.copy_(0.05 * torch.randn(203, 160, generator=g))
+    m = qa.mx_linear.from_linear(lin.cuda(), "int4d")
+    x = torch.randn(24, 160, generator=g).cuda().requires_grad_(True)
+    y = m(x)
+    go = torch.randn(24, 203, generator=g).cuda()
+    (gx,) = torch.autograd.grad(y, x, go)
+    wd = m.weight.cpu()
+    _check(y.detach().cpu(), x.detach().cpu(), wd, False)
+    _check(gx.cpu(), go.cpu(), wd, True)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.no_grad(), torch.cuda.stream(s):
+        m(x)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            yg = m(x)
+    torch.cuda.current_stream().wait_stream(s)
+    for _ in range(3):
+        yg.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(yg, y)
+        m(x)
