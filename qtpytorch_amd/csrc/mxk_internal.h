@@ -670,6 +670,17 @@ __device__ __forceinline__ float decode_field(uint32_t word, int sh, float s, co
 bool vec_rows_i32(const void* x, int x_type, int64_t rows, int64_t cols, int bits, int32_t* codes, float* scales,
                   hipStream_t st);
 
+// Hadamard rotation of rows of 129 .. 8192 elements (mxk_rot.hip): to fp32, or
+// fused with the quantizer / decoder of blocks of 128 (MXK_EUNSUPPORTED with
+// nothing launched for what the fused kernels do not take).
+bool rot_fits(int64_t d);
+int rot_rows(const void* in, int x_type, bool fwd, float* out, int64_t rows, int64_t d, const float* signs,
+             hipStream_t st);
+int rot_quantize(const void* x, int x_type, int64_t n, int64_t d, int mode, int bits, int block, const float* signs,
+                 uint8_t* packed, float* scales, int64_t n_store, float qf, hipStream_t st);
+int rot_dequantize(const uint8_t* packed, int64_t packed_nbytes, const float* scales, int64_t nb, int64_t n, int64_t d,
+                   int mode, int bits, int block, const float* signs, float* out, hipStream_t st);
+
 // MFMA weight-only linear (mxk_linear_mfma.hip) for int4/int8 weights with
 // blocks of 128 and N a multiple of 128: [K][N] weights (mx_linear) and
 // [N][K] weights (K a multiple of 128).  Workspace bytes (0 when the shape is

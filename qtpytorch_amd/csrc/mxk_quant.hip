@@ -622,7 +622,8 @@ __global__ __launch_bounds__(256) void k_quant_had128(const T* __restrict__ x, i
   }
 }
 
-// Generic rotation: one workgroup per row, n = next_pow2(d) <= 8192 in LDS.
+// Rotation of short rows: one workgroup per row, n = next_pow2(d) <= 128 in LDS
+// (longer rows: mxk_rot.hip).
 // FWD: out[r, :d] = (WHT(pad(x[r]) * signs) / sqrt(n))[:d]
 // INV: out[r, :d] = (WHT(pad(x[r])) / sqrt(n) * signs)[:d]
 template <typename T, bool FWD>
@@ -1208,7 +1209,11 @@ static int rotate_rows(const T* in, float* rot, int64_t rows, int64_t d, const f
   while ((int64_t(1) << logn) < n) ++logn;
   const float rdiv = (float)std::sqrt((double)n);
   const float rinv = 1.0f / rdiv;
-  if (n <= 8192) {
+  if (rot_fits(d)) {
+    const int xt = std::is_same<T, float>::value ? MXK_IN_F32 : std::is_same<T, __half>::value ? MXK_IN_F16 : MXK_IN_BF16;
+    return rot_rows(in, xt, FWD, rot, rows, d, signs, st);
+  }
+  if (n <= 128) {
     const int grid = (int)std::min<int64_t>(rows, (int64_t)num_cus() * 8);
     hipLaunchKernelGGL((k_fwht_rows<T, FWD>), dim3(std::max(grid, 1)), dim3(256), n * sizeof(float), st, in, rot, rows,
                        d, (int)n, logn, signs, rdiv, rinv);
@@ -1364,6 +1369,9 @@ int mxk_quantize(const void* x, int x_type, int64_t n, int kind, int bits, int v
       else ok = try_had128<hip_bfloat16>((const hip_bfloat16*)x, n, mode, bits, signs, pk, packed_nbytes, n_store, scales, qf, st);
       if (ok) return check_launch("quantize(hadamard128)");
     }
+    // longer rows of whole blocks: rotated and quantized in one kernel
+    const int frc = rot_quantize(x, x_type, n, rot_dim, mode, bits, block, signs, pk, scales, n_store, qf, st);
+    if (frc != MXK_EUNSUPPORTED) return frc;
     // rotate into the workspace, then quantize the float32 rotated copy
     const size_t need = mxk_quantize_workspace(n, kind, bits, variant, block, rot_dim);
     if (!workspace || workspace_nbytes < need) return fail(MXK_EINVAL, "quantize: workspace too small");
@@ -1412,6 +1420,11 @@ int mxk_dequantize(const void* packed, int64_t packed_nbytes, const float* scale
     MXK_DH(Q_FP, 4)
     MXK_DH(Q_FP, 8)
 #undef MXK_DH
+  }
+  if (variant == MXK_VAR_HADAMARD && signs && rot_dim > 0) {
+    const int frc = rot_dequantize(reinterpret_cast<const uint8_t*>(packed), packed_nbytes, scales, nb, n, rot_dim, mode,
+                                   bits, block, signs, out, st);
+    if (frc != MXK_EUNSUPPORTED) return frc;
   }
   int rc = MXK_EUNSUPPORTED;
 #define MXK_D(MODE, BITS) \
