@@ -1207,6 +1207,7 @@ struct GemmPlan {
   int KB, BP;
   int64_t KBP, Mpad, Npad;
   bool direct_a, v2, v3;
+  MidPlan mid;         // mxk_gemm_mid.hip
   bool small = false;  // k_qgemm_small: int8, block 128 or 64, grids of 256x128 tiles below the CU count
   int kn;  // 1: int8 with B read as stored, 2: int4 A and B read as stored (k_qgemm_kn), 0: unpacking pre-pass
   int req;  // output width requantized in the GEMM's epilogue (kn, N % 128 == 0), 0: a second pass
@@ -1249,6 +1250,15 @@ static GemmPlan plan_gemm(int64_t M, int64_t K, int64_t N, int bits, int block, 
     p.sa_bytes = up((size_t)p.KB * (size_t)M * sizeof(float));
     p.su_bytes = p.kn == 2 ? p.sa_bytes + 256 : 0;  // unscaled SA and the exact flag
     p.sb_bytes = up((size_t)p.KB * (size_t)N * sizeof(float));
+    return p;
+  }
+  // middle sizes, blocks of 64 and rows not on 16 bytes: one launch on the
+  // operands and scales as stored, requantizing in its epilogue where it can
+  if (aligned) p.mid = plan_mid(M, K, N, bits, block, out_bits);
+  if (p.mid.tm) {
+    p.direct_a = true;
+    p.v2 = p.v3 = false;
+    p.a_bytes = p.b_bytes = p.sa_bytes = p.sb_bytes = p.su_bytes = 0;
     return p;
   }
   // small int8 shapes: one launch on the operands and scales as stored
@@ -1432,6 +1442,16 @@ int mxk_qgemm(const void* a_packed, const float* a_scales, int64_t a_nscales, co
       return requant_vec_f32(Cb, M * N, out_bits, block, c_packed, c_packed_nbytes, c_scales, M * N, qw, p.q_bytes,
                              st);
     return MXK_OK;
+  }
+  if (p.mid.tm) {
+    const bool req = p.mid.req && aligned16(c_packed) && !acc_i32;
+    float* Cb = c_f32 ? c_f32 : (out_bits > 0 && !req ? reinterpret_cast<float*>(ws) : nullptr);
+    if (!Cb && !acc_i32 && !req) return fail(MXK_EINVAL, "qgemm: no output requested");
+    const int rc = run_mid(p.mid, a_packed, a_scales, a_ok, b_packed, b_scales, b_ok, M, K, N, bits, block, req,
+                           c_packed, c_scales, Cb, acc_i32, st);
+    if (rc != MXK_OK || out_bits <= 0 || req) return rc;
+    return requant_vec_f32(Cb, M * N, out_bits, block, c_packed, c_packed_nbytes, c_scales, M * N, ws + p.c_bytes,
+                           p.q_bytes, st);
   }
   if (p.small) {
     float* Cb = c_f32 ? c_f32 : (p.c_bytes ? reinterpret_cast<float*>(ws) : nullptr);

@@ -670,6 +670,17 @@ __device__ __forceinline__ float decode_field(uint32_t word, int sh, float s, co
 bool vec_rows_i32(const void* x, int x_type, int64_t rows, int64_t cols, int bits, int32_t* codes, float* scales,
                   hipStream_t st);
 
+// Packed GEMM of middle sizes (mxk_gemm_mid.hip): tm = 0 for what it does not
+// take; req: the requantization may run in its epilogue
+struct MidPlan {
+  int tm = 0;
+  bool req = false;
+};
+MidPlan plan_mid(int64_t M, int64_t K, int64_t N, int bits, int block, int out_bits);
+int run_mid(const MidPlan& p, const void* a, const float* sa, int a_ok, const void* b, const float* sb, int b_ok,
+            int64_t M, int64_t K, int64_t N, int bits, int block, bool req, void* cq, float* cq_scales, float* C,
+            int32_t* acc, hipStream_t st);
+
 // Hadamard rotation of rows of 129 .. 8192 elements (mxk_rot.hip): to fp32, or
 // fused with the quantizer / decoder of blocks of 128 (MXK_EUNSUPPORTED with
 // nothing launched for what the fused kernels do not take).
