@@ -466,10 +466,21 @@ __device__ __forceinline__ u32x4 qg3_unpack16(uint32_t w0, uint32_t w1) {
 //      layouts of mode 0 (A) and mode 1 (B).  Code c becomes the byte 16c
 //      (its nibble moved to the top of the byte: two instructions per four
 //      codes, no sign extension), so the MFMA sums P = sum (16a)(16b), 256
-//      times the code product.  sa_t then holds SA * 2^-8, and
-//      RN(float(P) * SA * 2^-8) = RN(P/256 * SA) when SA * 2^-8 is exact; with
-//      EXACT (some scale is too small for that) sa_t holds SA and P is
-//      scaled by 2^-8 first (exact: an integer below 2^24).
+//      times the code product.
+//
+// The epilogue of modes 1 and 2, three VALU instructions per output where a
+// conversion, two products and a sum take four.  The MFMAs sum onto 2^21, which
+// keeps every P + 2^21 in [0, 2^22], so that its bits are the float x = (P +
+// 2^21) 2^-149 (subnormal or in the lowest binade: evenly spaced, exact), and
+//   fma(x, S1, -S2),  S1 = SA 2^74 (int4: 2^66), S2 = S1 2^-128 = S1 2^21 2^-149
+// is RN(P SA) 2^-75 in one rounding (int4: the factor 256 of P is in S1); SB
+// 2^75 takes the power of two back out, and RN(RN(P SA) SB) and the sum onto C
+// keep their bits.  That needs SA = 0 or 2^-51 <= |SA| < 2^54 (RN(P SA) 2^-75
+// stays normal) and |SB| < 2^53; the quantizers' scales lie there.  k_prep_scales
+// checks every scale, and when one is outside, EXACT runs the four instructions
+// on SA itself (int4: P 2^-8 first, an exact integer).  8192^3:
+// int4 884 -> 800 us, int8 785 -> 772 us (with the loop's loads out of their
+// branches, below; int8 waits on its operands: the L2 delivers 8.5 TB/s).
 //
 // REQ (16 or 8): the requantization of C to REQ-bit codes by the 'v' rule
 // (mxtorch.py:1372-1385) runs in the epilogue, for N a multiple of 128:
@@ -487,6 +498,12 @@ __device__ __forceinline__ void qg3_run(int8_t* lds, const int8_t* __restrict__ 
                                         int grouped, const float* __restrict__ bias, uint8_t* __restrict__ cq = nullptr,
                                         float* __restrict__ cq_scales = nullptr) {
   static_assert(MODE == 0 || !ROWSCALE, "row scales are a mode-0 epilogue");
+  constexpr bool FMA3 = MODE != 0 && !EXACT;
+  i32x4 pinit = i32x4{0, 0, 0, 0};  // what the MFMAs of a block sum onto
+  if constexpr (FMA3) {
+    pinit = i32x4{1 << 21, 1 << 21, 1 << 21, 1 << 21};
+    asm volatile("" : "+v"(pinit));  // four registers, not four moves per tile
+  }
   // [A stages 0..2, 32 KiB each][B stages 0..2, 16 KiB each][scale stages 0..2, 2 KiB each]:
   // a stage's scales hold SA rows at floats 0..255 and SB columns at 256..383
   constexpr uint32_t LA = 0, LB = QG3_NS * 32768, LS = QG3_NS * (32768 + 16384);
@@ -637,11 +654,24 @@ __device__ __forceinline__ void qg3_run(int8_t* lds, const int8_t* __restrict__ 
   // (zeros before the first block: C + RN(RN(0*0)*0) = C for C = +0)
   i32x4 p3[4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
   i32x4 sa3 = {0, 0, 0, 0}, sb3 = {0, 0, 0, 0};
+  f32x4v sn3 = {0.0f, 0.0f, 0.0f, 0.0f};  // -S2 of sa3
+  auto minus_s2 = [&](const i32x4& sav) {
+    f32x4v r = {0.0f, 0.0f, 0.0f, 0.0f};
+    if constexpr (FMA3) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) r[i] = __int_as_float(sav[i]) * -0x1p-128f;
+    }
+    return r;
+  };
 
   // C = RN(C + RN(RN(P*SA)*SB)) for output (slice a, row i, fragment t) of K block kbw;
   // ROWSCALE (SA the same in every K block of a row): C = fma(P, SB, C), times SA at the end
-  auto epi_elem = [&](int a, int i, int t, const i32x4 (&p)[4], const i32x4& sav, const i32x4& sbvv, int kbw) {
-    if constexpr (ROWSCALE) {
+  auto epi_elem = [&](int a, int i, int t, const i32x4 (&p)[4], const i32x4& sav, const f32x4v& snv, const i32x4& sbvv,
+                      int kbw) {
+    if constexpr (FMA3) {
+      const float v = __builtin_fmaf(__int_as_float(p[t][i]), __int_as_float(sav[i]), snv[i]) * __int_as_float(sbvv[t]);
+      c[a][t][i] = c[a][t][i] + v;
+    } else if constexpr (ROWSCALE) {
       c[a][t][i] = __builtin_fmaf((float)p[t][i], __int_as_float(sbvv[t]), c[a][t][i]);
     } else {
       float pf = (float)p[t][i];
@@ -653,7 +683,7 @@ __device__ __forceinline__ void qg3_run(int8_t* lds, const int8_t* __restrict__ 
       const int64_t row = m0 + wm * 64 + a * 16 + lg * 4 + i;
       const int64_t col = n0 + wn * 64 + t * 16 + lcol;
       if (kbw >= 0 && row < M && col < N)
-        acc_out[((int64_t)kbw * M + row) * N + col] = MODE == 2 ? (p[t][i] >> 8) : p[t][i];
+        acc_out[((int64_t)kbw * M + row) * N + col] = (FMA3 ? p[t][i] - (1 << 21) : p[t][i]) >> (MODE == 2 ? 8 : 0);
     }
   };
 
@@ -669,15 +699,17 @@ __device__ __forceinline__ void qg3_run(int8_t* lds, const int8_t* __restrict__ 
     // (modes 0/1: its 7 loads; mode 2: the 3 packed loads and the scale load
     // of stage kb+1); mode 2 also waits for its own LDS stores of stage kb
     if constexpr (MODE == 2) {
-      if (kb + 1 < KB) wait_vmcnt<4>();
-      else wait_vmcnt<0>();
+      wait_vmcnt<4>();
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     } else {
-      if (kb + 1 < KB) wait_vmcnt<7>();
-      else wait_vmcnt<0>();
+      wait_vmcnt<7>();
     }
     qg3_barrier();  // stage kb visible; every wave is done with stage kb-1
-    const bool ld = kb + 2 < KB;
+    // Every stage issues its loads: past the last block they read it again,
+    // into a buffer that nobody reads.  With the loads behind `if`s each K
+    // block fell into five basic blocks, the compiler moved all of the
+    // epilogue into the last one, and MFMAs and VALU took turns.
+    const int kn = kb + 2 < KB ? kb + 2 : KB - 1;
     const int lbuf = cur == 0 ? 2 : cur - 1;
     // reads in need order, at most 15 in flight (the lgkmcnt limit): A
     // slice 0, B column fragments 0..3, SB, SA0, A slice 1, SA1
@@ -717,32 +749,33 @@ __device__ __forceinline__ void qg3_run(int8_t* lds, const int8_t* __restrict__ 
     auto slice_mfma = [&](int a, i32x4 (&p)[4]) {
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        p[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(af[a][0], bf[0][t], i32x4{0, 0, 0, 0}, 0, 0, 0);
+        p[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(af[a][0], bf[0][t], pinit, 0, 0, 0);
         p[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(af[a][1], bf[1][t], p[t], 0, 0, 0);
       }
     };
     auto slice_epilogue = [&](int a, const i32x4 (&p)[4], const i32x4& sav) {
+      const f32x4v snv = minus_s2(sav);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) epi_elem(a, i, t, p, sav, sbv, kb);
+        for (int t = 0; t < 4; ++t) epi_elem(a, i, t, p, sav, snv, sbv, kb);
     };
     // The MFMAs of slice a+1 go one by one between the epilogue VALU ops of
-    // slice a (8 MFMAs, 64 VALU ops), so the matrix core runs while the same
+    // slice a (8 MFMAs, 52 VALU ops; 64 without FMA3), so the matrix core runs while the same
     // wave issues the epilogue.
 #define QG3_INTERLEAVE()                                 \
     for (int ii = 0; ii < 8; ++ii) {                     \
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); \
-      __builtin_amdgcn_sched_group_barrier(0x002, 8, 0); \
+      __builtin_amdgcn_sched_group_barrier(0x002, FMA3 ? 7 : 8, 0); \
     }
     i32x4 p0[4], p1[4];
     // Slice 0: MFMA pair t waits only for its own fragments (A0 and B
     // column fragment t: the first 4 + 2t reads); the carried slice-3
-    // epilogue of the previous K block fills the gaps, 2 outputs (8 VALU
+    // epilogue of the previous K block fills the gaps, 2 outputs (6 or 8 VALU
     // ops) per chunk.
     auto chunk = [&](int j) {
-      epi_elem(3, (2 * j) >> 2, (2 * j) & 3, p3, sa3, sb3, kb - 1);
-      epi_elem(3, (2 * j + 1) >> 2, (2 * j + 1) & 3, p3, sa3, sb3, kb - 1);
+      epi_elem(3, (2 * j) >> 2, (2 * j) & 3, p3, sa3, sn3, sb3, kb - 1);
+      epi_elem(3, (2 * j + 1) >> 2, (2 * j + 1) & 3, p3, sa3, sn3, sb3, kb - 1);
     };
 #define QG3_SLICE0_PAIR(T, WAITN)                                                                   \
     chunk(2 * T);                                                                                   \
@@ -752,7 +785,7 @@ __device__ __forceinline__ void qg3_run(int8_t* lds, const int8_t* __restrict__ 
     qg3_lgkm_wait<WAITN>(bf[0][T]);                                                                 \
     qg3_lgkm_wait<WAITN>(bf[1][T]);                                                                 \
     __builtin_amdgcn_sched_barrier(0);                                                              \
-    p0[T] = __builtin_amdgcn_mfma_i32_16x16x64_i8(af[0][0], bf[0][T], i32x4{0, 0, 0, 0}, 0, 0, 0); \
+    p0[T] = __builtin_amdgcn_mfma_i32_16x16x64_i8(af[0][0], bf[0][T], pinit, 0, 0, 0);              \
     __builtin_amdgcn_sched_barrier(0);                                                              \
     chunk(2 * T + 1);                                                                               \
     __builtin_amdgcn_sched_barrier(0);                                                              \
@@ -771,7 +804,7 @@ __device__ __forceinline__ void qg3_run(int8_t* lds, const int8_t* __restrict__ 
     __builtin_amdgcn_sched_barrier(0);                                                              \
     bf[0][T] = i32x4{btr[T][0][0], btr[T][0][1], btr[T][1][0], btr[T][1][1]};                       \
     bf[1][T] = i32x4{btr[T][2][0], btr[T][2][1], btr[T][3][0], btr[T][3][1]};                       \
-    p0[T] = __builtin_amdgcn_mfma_i32_16x16x64_i8(af[0][0], bf[0][T], i32x4{0, 0, 0, 0}, 0, 0, 0); \
+    p0[T] = __builtin_amdgcn_mfma_i32_16x16x64_i8(af[0][0], bf[0][T], pinit, 0, 0, 0);              \
     __builtin_amdgcn_sched_barrier(0);                                                              \
     chunk(2 * T + 1);                                                                               \
     __builtin_amdgcn_sched_barrier(0);                                                              \
@@ -799,6 +832,10 @@ __device__ __forceinline__ void qg3_run(int8_t* lds, const int8_t* __restrict__ 
 #undef QG3_SLICE0_PAIR
 #undef QG3_SLICE0_PAIRT
     qg3_lgkm_wait<0>(sbv);
+    if constexpr (FMA3) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) sbv[t] = __float_as_int(__int_as_float(sbv[t]) * 0x1p75f);
+    }
     qg3_lgkm_wait<0>(sa[0]);
     qg3_lgkm_wait<0>(af[1][0]);
     qg3_lgkm_wait<0>(af[1][1]);
@@ -809,7 +846,7 @@ __device__ __forceinline__ void qg3_run(int8_t* lds, const int8_t* __restrict__ 
     af[3][0] = qg3_ds_read<3 * 2048>(b0);
     af[3][1] = qg3_ds_read<3 * 2048>(b1);
     sa[3] = qg3_ds_read<192>(bsa);
-    if (MODE != 2 && ld) load_part(kb + 2, lbuf, 0);
+    if constexpr (MODE != 2) load_part(kn, lbuf, 0);
     __builtin_amdgcn_sched_barrier(0);
     slice_mfma(1, p1);
     slice_epilogue(0, p0, sa[0]);
@@ -818,7 +855,7 @@ __device__ __forceinline__ void qg3_run(int8_t* lds, const int8_t* __restrict__ 
     qg3_lgkm_wait<3>(af[2][0]);
     qg3_lgkm_wait<3>(af[2][1]);
     qg3_lgkm_wait<3>(sa[2]);
-    if (MODE != 2 && ld) load_part(kb + 2, lbuf, 1);
+    if constexpr (MODE != 2) load_part(kn, lbuf, 1);
     __builtin_amdgcn_sched_barrier(0);
     slice_mfma(2, p0);
     slice_epilogue(1, p1, sa[1]);
@@ -832,14 +869,12 @@ __device__ __forceinline__ void qg3_run(int8_t* lds, const int8_t* __restrict__ 
       // during kb-1) into its buffer, then load stage kb+2 into the VGPRs
       // and its scales into the stage every wave finished before this
       // block's barrier
-      if (kb + 1 < KB) write4(cur == 2 ? 0 : cur + 1);
-      if (ld) {
-        load4(kb + 2);
-        load_part(kb + 2, lbuf, 3);
-      }
-    } else if (ld) {
-      load_part(kb + 2, lbuf, 2);
-      load_part(kb + 2, lbuf, 3);
+      write4(cur == 2 ? 0 : cur + 1);
+      load4(kn);
+      load_part(kn, lbuf, 3);
+    } else {
+      load_part(kn, lbuf, 2);
+      load_part(kn, lbuf, 3);
     }
     __builtin_amdgcn_sched_barrier(0);
     slice_mfma(3, p3);
@@ -848,39 +883,39 @@ __device__ __forceinline__ void qg3_run(int8_t* lds, const int8_t* __restrict__ 
     __builtin_amdgcn_sched_barrier(0);
 #undef QG3_INTERLEAVE
     sa3 = sa[3];
+    sn3 = minus_s2(sa3);
     sb3 = sbv;
   };
 
+  const int k1 = KB > 1 ? 1 : 0;
   if constexpr (MODE == 2) {
     // stage 0 unpacked into LDS, stage 1 in flight (packed codes in VGPRs)
     load4(0);
     load_part(0, 0, 3);
     write4(0);
-    if (KB > 1) {
-      load4(1);
-      load_part(1, 1, 3);
-    }
+    load4(k1);
+    load_part(k1, 1, 3);
   } else {
     load_part(0, 0, 0);
     load_part(0, 0, 1);
     load_part(0, 0, 2);
     load_part(0, 0, 3);
-    if (KB > 1) {
-      load_part(1, 1, 0);
-      load_part(1, 1, 1);
-      load_part(1, 1, 2);
-      load_part(1, 1, 3);
-    }
+    load_part(k1, 1, 0);
+    load_part(k1, 1, 1);
+    load_part(k1, 1, 2);
+    load_part(k1, 1, 3);
   }
   int cur = 0;
   for (int kb = 0; kb < KB; ++kb) {
     body(kb, cur);
     cur = cur == 2 ? 0 : cur + 1;
   }
+  wait_vmcnt<0>();  // the last blocks' loads to LDS
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int t = 0; t < 4; ++t) epi_elem(3, i, t, p3, sa3, sb3, KB - 1);
+    for (int t = 0; t < 4; ++t) epi_elem(3, i, t, p3, sa3, sn3, sb3, KB - 1);
   if (WRITE_C) {
 #pragma unroll
     for (int a = 0; a < 4; ++a)
@@ -957,19 +992,21 @@ __global__ __launch_bounds__(512, 1) void k_qgemm_i8_v3(const int8_t* __restrict
 }
 
 // The packed GEMM on operands as the caller stores them: mode 1 (int8; B
-// [K][N]) or mode 2 (int4; A [M][K/2], B [K][N/2]), see qg3_run.  Mode 2
-// reads `exact` (written by k_prep_sa4) once: 0 takes sa_s = SA * 2^-8, 1
-// the exact epilogue on sa_u = SA.
+// [K][N]) or mode 2 (int4; A [M][K/2], B [K][N/2]), see qg3_run.  `flags`
+// (QG_PREP_WGS of them, written by k_prep_scales): all zero takes the three-
+// instruction epilogue on sa_s = S1, any other the exact one on sa_u = SA.
+#define QG_PREP_WGS 512
 template <int MODE, bool WRITE_ACC, bool WRITE_C, int REQ = 0>
 __global__ __launch_bounds__(512, 1) void k_qgemm_kn(const int8_t* __restrict__ A, int64_t lda, int64_t Arows,
                                                      const int8_t* __restrict__ B, int64_t ldb, int64_t Brows,
                                                      const float* __restrict__ sa_s, const float* __restrict__ sa_u,
-                                                     const int* __restrict__ exact, const float* __restrict__ sb_src,
+                                                     const int* __restrict__ flags, const float* __restrict__ sb_src,
                                                      int64_t M, int64_t N, int KB, float* __restrict__ C,
                                                      int32_t* __restrict__ acc_out, int grouped,
                                                      uint8_t* __restrict__ cq, float* __restrict__ cq_scales) {
   __shared__ __attribute__((aligned(1024))) int8_t lds[QG3_LDS_BYTES];
-  if (MODE == 2 && __builtin_amdgcn_readfirstlane(*exact) != 0)
+  static_assert(QG_PREP_WGS == 512, "a flag per thread");
+  if (__syncthreads_or(flags[threadIdx.x]) != 0)
     qg3_run<MODE, WRITE_ACC, WRITE_C, false, true, REQ>(lds, A, lda, Arows, B, ldb, Brows, sa_u, sb_src, M, N, KB, C,
                                                         acc_out, grouped, nullptr, cq, cq_scales);
   else
@@ -1157,36 +1194,47 @@ __global__ __launch_bounds__(256) void k_transpose_sa(const float* __restrict__ 
   }
 }
 
-// The int4 loop's A scales: ts[kb][m] = SA * 2^-8 and tu[kb][m] = SA for SA
-// = s[m * KB + kb] (1 when s is null); *exact becomes 1 when some SA * 2^-8
-// is inexact (an SA below 2^-118 with low bits that the shift drops), which
-// selects the loop's exact epilogue.  *exact is zeroed by k_zero_flag first.
-__global__ __launch_bounds__(256) void k_prep_sa4(const float* __restrict__ s, int64_t M, int64_t KB,
-                                                  float* __restrict__ ts, float* __restrict__ tu,
-                                                  int* __restrict__ exact) {
-  __shared__ float tile[32][33];
-  const int64_t k0 = (int64_t)blockIdx.x * 32, m0 = (int64_t)blockIdx.y * 32;
-  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-  for (int i = ty; i < 32; i += 8) {
-    const int64_t m = m0 + i, k = k0 + tx;
-    tile[i][tx] = (m < M && k < KB) ? (s ? s[m * KB + k] : 1.0f) : 0.0f;
-  }
-  __syncthreads();
-  bool lost = false;
-  for (int i = ty; i < 32; i += 8) {
-    const int64_t k = k0 + i, m = m0 + tx;
-    if (k < KB && m < M) {
-      const float v = tile[tx][i];
-      const float vs = v * 0.00390625f;
-      ts[k * M + m] = vs;
-      tu[k * M + m] = v;
-      lost = lost || (vs * 256.0f != v && v == v);
+// The scales of the as-stored loops: ts[kb][m] = SA * f (f = 2^74, or 2^66 for
+// int4) and tu[kb][m] = SA for SA = s[m * KB + kb] (1 when s is null), by the
+// first QG_PREP_WGS - 64 workgroups; the other 64 read SB.  Each workgroup
+// writes whether it met a scale that the three-instruction epilogue does not
+// take (qg3_run) into its own flag: nothing to clear first.
+__global__ __launch_bounds__(256) void k_prep_scales(const float* __restrict__ s, int64_t M, int64_t KB, float f,
+                                                     const float* __restrict__ sb, int64_t nsb, float* __restrict__ ts,
+                                                     float* __restrict__ tu, int* __restrict__ flags) {
+  constexpr int WGB = 64, WGA = QG_PREP_WGS - WGB;
+  bool out = false;
+  if (blockIdx.x >= WGA) {
+    const int64_t stride = (int64_t)WGB * 256;
+#pragma unroll 4
+    for (int64_t i = (int64_t)(blockIdx.x - WGA) * 256 + threadIdx.x; i < nsb; i += stride)
+      out = out || !(__builtin_fabsf(sb[i]) < 0x1p53f);
+  } else {
+    __shared__ float tile[32][33];
+    const int64_t tk = (KB + 31) / 32, tm = (M + 31) / 32;
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    for (int64_t b = blockIdx.x; b < tk * tm; b += WGA) {
+      const int64_t k0 = (b % tk) * 32, m0 = (b / tk) * 32;
+      for (int i = ty; i < 32; i += 8) {
+        const int64_t m = m0 + i, k = k0 + tx;
+        tile[i][tx] = (m < M && k < KB) ? (s ? s[m * KB + k] : 1.0f) : 0.0f;
+      }
+      __syncthreads();
+      for (int i = ty; i < 32; i += 8) {
+        const int64_t k = k0 + i, m = m0 + tx;
+        if (k < KB && m < M) {
+          const float v = tile[tx][i], a = __builtin_fabsf(v);
+          ts[k * M + m] = v * f;
+          tu[k * M + m] = v;
+          out = out || !(v == 0.0f || (a >= 0x1p-51f && a < 0x1p54f));
+        }
+      }
+      __syncthreads();
     }
   }
-  if (lost) atomicOr(exact, 1);
+  const int any = __syncthreads_or(out);
+  if (threadIdx.x == 0) flags[blockIdx.x] = any != 0;
 }
-
-__global__ void k_zero_flag(int* __restrict__ p) { *p = 0; }
 
 // t[kb][r] (kb_major) or t[r][kb] = s[(r*K + kb*kblk) / B]: the scale of
 // the kblk-wide K chunk kb of row r of a [R][K] operand whose flat blocks
@@ -1248,7 +1296,7 @@ static GemmPlan plan_gemm(int64_t M, int64_t K, int64_t N, int bits, int block, 
     p.v2 = p.v3 = true;
     p.a_bytes = p.b_bytes = 0;
     p.sa_bytes = up((size_t)p.KB * (size_t)M * sizeof(float));
-    p.su_bytes = p.kn == 2 ? p.sa_bytes + 256 : 0;  // unscaled SA and the exact flag
+    p.su_bytes = p.sa_bytes + QG_PREP_WGS * sizeof(int);  // unscaled SA and the flags
     p.sb_bytes = up((size_t)p.KB * (size_t)N * sizeof(float));
     return p;
   }
@@ -1375,27 +1423,18 @@ int mxk_qgemm(const void* a_packed, const float* a_scales, int64_t a_nscales, co
   const int a_ok = a_nscales == M * p.KB;
   const int b_ok = b_nscales == (int64_t)p.KB * N;
   if (p.kn) {
-    // operands as stored: no unpacking or transposing pass
+    // operands as stored: no unpacking or transposing pass over them
     float* Cb = c_f32 ? c_f32 : (p.c_bytes ? reinterpret_cast<float*>(ws) : nullptr);
     void* qw = ws + p.c_bytes;
     float* sa_s = reinterpret_cast<float*>(ws + p.c_bytes + p.q_bytes);
     float* sb_one = reinterpret_cast<float*>(ws + p.c_bytes + p.q_bytes + p.sa_bytes);
-    float* sa_u = p.kn == 2 ? reinterpret_cast<float*>(ws + p.c_bytes + p.q_bytes + p.sa_bytes + p.sb_bytes)
-                            : nullptr;
-    int* exact = p.kn == 2 ? reinterpret_cast<int*>(reinterpret_cast<uint8_t*>(sa_u) + p.sa_bytes) : nullptr;
+    float* sa_u = reinterpret_cast<float*>(ws + p.c_bytes + p.q_bytes + p.sa_bytes + p.sb_bytes);
+    int* flags = reinterpret_cast<int*>(reinterpret_cast<uint8_t*>(sa_u) + p.sa_bytes);
     if (!Cb && !acc_i32 && !p.req) return fail(MXK_EINVAL, "qgemm: no output requested");
     const int cap = num_cus() * 8;
-    const dim3 tg((unsigned)ceil_div(p.KB, 32), (unsigned)ceil_div(M, 32));
-    if (p.kn == 2) {
-      hipLaunchKernelGGL(k_zero_flag, dim3(1), dim3(1), 0, st, exact);
-      hipLaunchKernelGGL(k_prep_sa4, tg, dim3(256), 0, st, a_ok ? a_scales : nullptr, M, (int64_t)p.KB, sa_s, sa_u,
-                         exact);
-    } else if (a_ok) {
-      hipLaunchKernelGGL(k_transpose_sa, tg, dim3(256), 0, st, a_scales, M, (int64_t)p.KB, sa_s);
-    } else {
-      hipLaunchKernelGGL(k_fill_ones, dim3((unsigned)std::min<int64_t>(ceil_div((int64_t)p.KB * M, 256), cap)),
-                         dim3(256), 0, st, sa_s, (int64_t)p.KB * M);
-    }
+    hipLaunchKernelGGL(k_prep_scales, dim3(QG_PREP_WGS), dim3(256), 0, st, a_ok ? a_scales : nullptr, M,
+                       (int64_t)p.KB, p.kn == 2 ? 0x1p66f : 0x1p74f, b_scales, b_ok ? (int64_t)p.KB * N : (int64_t)0,
+                       sa_s, sa_u, flags);
     const float* sbs = b_scales;
     if (!b_ok) {
       hipLaunchKernelGGL(k_fill_ones, dim3((unsigned)std::min<int64_t>(ceil_div((int64_t)p.KB * N, 256), cap)),
@@ -1409,7 +1448,7 @@ int mxk_qgemm(const void* a_packed, const float* a_scales, int64_t a_nscales, co
     const int8_t* B = (const int8_t*)b_packed;
     const int64_t lda = p.kn == 2 ? K / 2 : K, ldb = p.kn == 2 ? N / 2 : N;
 #define QG_KN_LAUNCH(MODE, WA, WC, REQ)                                                                         \
-  hipLaunchKernelGGL((k_qgemm_kn<MODE, WA, WC, REQ>), g1, dim3(512), 0, st, A, lda, M, B, ldb, K, sa_s, sa_u, exact, \
+  hipLaunchKernelGGL((k_qgemm_kn<MODE, WA, WC, REQ>), g1, dim3(512), 0, st, A, lda, M, B, ldb, K, sa_s, sa_u, flags, \
                      sbs, M, N, p.KB, Cb, acc_i32, grouped, (uint8_t*)c_packed, c_scales)
     if (p.req) {
       // c_f32 and acc_i32 (when asked for) are written as well; no workspace C, no second pass
