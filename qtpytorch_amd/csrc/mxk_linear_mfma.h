@@ -185,12 +185,21 @@ __device__ __forceinline__ void lm_put(float* __restrict__ xs, _Float16* __restr
   }
 }
 
+// The row that workgroup b of the row pass takes: the 16 rows of a row tile go to
+// one XCD (workgroup b runs on XCD b % 8), since every 128-byte line of the
+// tiled layout holds 16 bytes of each of 8 of them: with row b on XCD b % 8,
+// eight L2s wrote pieces of each line (2048 x 4096 bf16: 31 -> 11.5 us with no lo
+// to write either; fp32 x to fp32 22 -> 15.5 us).
+__device__ __forceinline__ int64_t lm_prep_m(int64_t b, int64_t M) {
+  return b < (M & ~(int64_t)127) ? (b & ~(int64_t)127) + (b & 7) * 16 + ((b >> 3) & 15) : b;
+}
+
 // Row m by one workgroup of 256 threads (red: 4 floats of LDS)
 template <typename T, bool SPLIT, bool VEC, bool LO = true>
 __device__ __forceinline__ void lm_prep_row(const T* __restrict__ x, int64_t m, int64_t K, int64_t Kp,
                                             float* __restrict__ xs, _Float16* __restrict__ xh,
                                             _Float16* __restrict__ xl, int* __restrict__ ex, float* red) {
-  static_assert(LO || sizeof(T) == 2, "fp32 x needs lo");
+  static_assert(LO || (SPLIT && sizeof(T) == 2), "fp32 x needs lo");
   constexpr int E = 16 / (int)sizeof(T), NCH = 8;
   const int tid = threadIdx.x;
   const T* row = x + m * K;
@@ -267,7 +276,7 @@ __device__ __forceinline__ void lm_prep_row(const T* __restrict__ x, int64_t m, 
 // the block-major scales sT [NB][K]) in [2^13, 2^14), 0 for a zero or
 // non-finite maximum.  It depends on the weight alone; computed here, it is
 // ready before the main kernel starts.
-template <typename T, bool SPLIT, bool VEC>
+template <typename T, bool SPLIT, bool VEC, bool LO>
 __global__ __launch_bounds__(256) void k_linear_mfma_prep_rows(const T* __restrict__ x, int64_t M, int64_t K,
                                                                int64_t Kp, float* __restrict__ xs,
                                                                _Float16* __restrict__ xh, _Float16* __restrict__ xl,
@@ -298,7 +307,7 @@ __global__ __launch_bounds__(256) void k_linear_mfma_prep_rows(const T* __restri
     }
     return;
   }
-  lm_prep_row<T, SPLIT, VEC>(x, (int64_t)blockIdx.x, K, Kp, xs, xh, xl, ex, red);
+  lm_prep_row<T, SPLIT, VEC, LO>(x, lm_prep_m(blockIdx.x, M), K, Kp, xs, xh, xl, ex, red);
 }
 
 inline size_t lm_round(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -307,12 +316,14 @@ inline size_t lm_round(size_t v) { return (v + 255) & ~(size_t)255; }
 template <typename T, bool SPLIT>
 void lm_prep_rows_t(const T* x, int64_t M, int64_t K, int64_t Kp, float* xs, _Float16* xh, _Float16* xl, int* ex,
                     const float* sT, int64_t NB, int* es, hipStream_t st) {
+  // 16-bit x has no lo part (lm_put)
+  constexpr bool LO = !SPLIT || sizeof(T) == 4;
   const dim3 grid((unsigned)(M + (sT ? NB : 0)));
   if (aligned16(x) && (K * (int64_t)sizeof(T)) % 16 == 0)
-    hipLaunchKernelGGL((k_linear_mfma_prep_rows<T, SPLIT, true>), grid, dim3(256), 0, st, x, M, K, Kp, xs, xh, xl, ex,
+    hipLaunchKernelGGL((k_linear_mfma_prep_rows<T, SPLIT, true, LO>), grid, dim3(256), 0, st, x, M, K, Kp, xs, xh, xl, ex,
                        sT, es);
   else
-    hipLaunchKernelGGL((k_linear_mfma_prep_rows<T, SPLIT, false>), grid, dim3(256), 0, st, x, M, K, Kp, xs, xh, xl,
+    hipLaunchKernelGGL((k_linear_mfma_prep_rows<T, SPLIT, false, LO>), grid, dim3(256), 0, st, x, M, K, Kp, xs, xh, xl,
                        ex, sT, es);
 }
 

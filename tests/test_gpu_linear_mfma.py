@@ -358,3 +358,21 @@ def test_mx_linear_rotated_and_vector_weights(qa, dt):
         w_f = orc.dequant(wp, ws, dt, K * N, 128, orig_shape=(K, N), hadamard_mode=mode).reshape(K, N)
         ok, worst = _rowwise(y, x @ w_f)
         assert ok, f"{dt} ({mode}): worst row error {worst:.3g} x the bar"
+
+
+@pytest.mark.parametrize("dt", ["int4d", "int8d", "float8d"])
+@pytest.mark.parametrize("src", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M", [17, 130, 300])
+def test_16_bit_x_is_its_own_hi(qa, dt, src, M):
+    """[out, in] weights: fp16 and bf16 x take one product per term.  Their
+    scaled values are their own f16 hi, so the result is the fp32 path's bits,
+    also for values far below a row's largest."""
+    K, N = 384, 256
+    x = _randn((M, K), 31 + M) * 10.0 ** torch.linspace(-4, 4, M)[:, None]
+    x[:, ::7] *= 2.0 ** -13
+    x[:, 1::7] *= 2.0 ** -26
+    x = x.to(src)
+    w = 0.02 * _randn((N, K), 5)
+    q = qa.mx_tensor.quantize(w.to(dev()), dt, 128)
+    args = (q._mx_packed, q._mx_scales, q._mx_dtype, N, K, 128)
+    assert torch.equal(qa.ops.linear_wq_nt(x.to(dev()), *args), qa.ops.linear_wq_nt(x.float().to(dev()), *args))
