@@ -557,14 +557,15 @@ __device__ __forceinline__ void qg3_run(int8_t* lds, const int8_t* __restrict__ 
   }
   const int f = 64 * wave + lane;
   // waves 0-3: SA rows, 4-5: SB columns, 6-7: a harmless load of SA row 0
-  const bool is_b = wave == 4 || wave == 5;
+  // (ROWSCALE has no scale per row and block: sb_src there too, sa_t is [M])
+  const bool is_b = ROWSCALE || wave == 4 || wave == 5;
   const float* gsb = is_b ? sb_src : sa_t;
   const int64_t gstride = is_b ? N : M;
   // SB is stored lane-major: float 256 + 64*wn + 4*lr + t holds column
   // n0 + 64*wn + 16t + qg3_lcol(lr), so a lane's four SB values are one 16-byte read
   const int fb = f - 256;  // 0..127 on waves 4-5
   const uint32_t os =
-      (uint32_t)(4 * (f < 256 ? std::min<int64_t>(m0 + f, M - 1)
+      (uint32_t)(4 * (f < 256 ? (ROWSCALE ? 0 : std::min<int64_t>(m0 + f, M - 1))
                               : (f < 384 ? std::min<int64_t>(n0 + (fb & ~63) + (fb & 3) * 16 +
                                                                  qg3_lcol<MODE>((fb & 63) >> 2),
                                                              N - 1)
@@ -1653,19 +1654,32 @@ int mxk_linear_i8(const void* x_packed, int64_t x_nbytes, const float* x_scales,
                        (const uint8_t*)w_packed, w_nbytes, w_bits, N, p.Npad, K, K, 1, p.kblk, p.kblk, p.KB,
                        (int8_t*)B8);
   }
-  // SA: [KB][M] for v2/v3, [M][KB] for the one-stage kernel; SB: [KB][N]
-  hipLaunchKernelGGL(k_gather_scales, dim3((unsigned)std::min<int64_t>(ceil_div(M * p.KB, 256), cap)), dim3(256), 0,
-                     st, x_scales, x_nscales, M, K, x_block, p.kblk, p.KB, p.v2 ? 1 : 0, sa);
-  hipLaunchKernelGGL(k_gather_scales, dim3((unsigned)std::min<int64_t>(ceil_div(N * p.KB, 256), cap)), dim3(256), 0,
-                     st, w_scales, w_nscales, N, K, w_block, p.kblk, p.KB, 1, sb);
+  // SA: [KB][M] for v2/v3, [M][KB] for the one-stage kernel; SB: [KB][N].
+  // Per-token x in the large loop takes one scale a row, as stored; the scales
+  // of blocks of 128 are a plain transpose (4000 x 4096 x 4096: two gathers of
+  // 4.8 us -> one transpose of 4.8 us, whose time is the launch's).
+  const bool rowscale = p.v3 && x_block % K == 0;
+  const float* sa_row = x_block == K ? x_scales : sa;
+  if (!rowscale)
+    hipLaunchKernelGGL(k_gather_scales, dim3((unsigned)std::min<int64_t>(ceil_div(M * p.KB, 256), cap)), dim3(256), 0,
+                       st, x_scales, x_nscales, M, K, x_block, p.kblk, p.KB, p.v2 ? 1 : 0, sa);
+  else if (x_block != K)
+    hipLaunchKernelGGL(k_gather_scales, dim3((unsigned)std::min<int64_t>(ceil_div(M, 256), cap)), dim3(256), 0, st,
+                       x_scales, x_nscales, M, K, x_block, (int)std::min<int64_t>(K, INT32_MAX), 1, 1, sa);
+  if (w_block == p.kblk && ceil_div(N, 32) < 65536)
+    hipLaunchKernelGGL(k_transpose_sa, dim3((unsigned)ceil_div(p.KB, 32), (unsigned)ceil_div(N, 32)), dim3(256), 0, st,
+                       w_scales, N, (int64_t)p.KB, sb);
+  else
+    hipLaunchKernelGGL(k_gather_scales, dim3((unsigned)std::min<int64_t>(ceil_div(N * p.KB, 256), cap)), dim3(256), 0,
+                       st, w_scales, w_nscales, N, K, w_block, p.kblk, p.KB, 1, sb);
   const int64_t arows = p.direct_x ? M : p.Mpad, brows = p.direct_w ? N : p.Npad;
   if (p.v3) {
     const int64_t tiles_m = ceil_div(M, QG3_BM), tiles_n = ceil_div(N, QG3_BN);
     const int grouped = (tiles_m % 8 == 0 && tiles_n % 8 == 0 && (tiles_m * tiles_n) % 512 == 0) ? 1 : 0;
     // per-token activations (one x scale per row): the row scale leaves the K loop
-    if (x_block % K == 0)
+    if (rowscale)
       hipLaunchKernelGGL((k_qgemm_i8_v3<false, true, true>), dim3((unsigned)(tiles_m * tiles_n)), dim3(512), 0, st,
-                         A8, K, arows, B8, K, brows, sa, sb, M, N, p.KB, out, nullptr, grouped, bias);
+                         A8, K, arows, B8, K, brows, sa_row, sb, M, N, p.KB, out, nullptr, grouped, bias);
     else
       hipLaunchKernelGGL((k_qgemm_i8_v3<false, true>), dim3((unsigned)(tiles_m * tiles_n)), dim3(512), 0, st, A8, K,
                          arows, B8, K, brows, sa, sb, M, N, p.KB, out, nullptr, grouped, bias);
