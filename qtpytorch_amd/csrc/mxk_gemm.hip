@@ -1345,6 +1345,8 @@ struct I8LinPlan {
   bool direct_x, direct_w, v2, v3;
   int64_t Mpad, Npad;
   size_t x_bytes, w_bytes, sa_bytes, sb_bytes;
+  MidLin mid;          // mxk_gemm_mid.hip
+  size_t part_bytes;   // its partial sums: where the workspace ends before them, K is not split
 };
 
 static I8LinPlan plan_i8lin(int64_t M, int64_t K, int64_t N, int xbits, int wbits, int64_t xb, int64_t wb) {
@@ -1366,7 +1368,14 @@ static I8LinPlan plan_i8lin(int64_t M, int64_t K, int64_t N, int xbits, int wbit
   const int64_t lim = (int64_t)1 << 31;
   const bool fits32 = (p.direct_x ? M : p.Mpad) * K < lim && (p.direct_w ? N : p.Npad) * K < lim &&
                       (int64_t)p.KB * M * 4 < lim && (int64_t)p.KB * N * 4 < lim;
-  p.v3 = p.v2 && fits32 && ceil_div(M, QG3_BM) * ceil_div(N, QG3_BN) >= num_cus();
+  if (xbits == wbits) p.mid = plan_mid_lin(M, K, N, xbits, xb, wb, p.kblk);
+  // past the 64-tiles the 256 x 128 loop wins before it fills the chip
+  // (192 tiles, 1500x4096x4096: 64.0 -> 52.2 us), unless K is short
+  // (200x512x28000: 21.3 -> 22.2)
+  p.v3 = p.v2 && fits32 &&
+         ((K >= 1024 && ceil_div(M, 64) * ceil_div(N, 64) > 4 * num_cus()) ||
+          ceil_div(M, QG3_BM) * ceil_div(N, QG3_BN) >= num_cus());
+  p.part_bytes = p.mid.splits > 1 ? up((size_t)p.mid.splits * (size_t)M * (size_t)N * sizeof(float)) : 0;
   return p;
 }
 
@@ -1611,7 +1620,7 @@ size_t mxk_linear_i8_workspace(int64_t M, int64_t K, int64_t N, int x_bits, int 
   if (M <= 0 || K <= 0 || N <= 0 || x_block <= 0 || w_block <= 0) return 0;
   I8LinPlan p = plan_i8lin(M, K, N, x_bits, w_bits, x_block, w_block);
   if (p.kblk == 0) return 0;
-  return p.x_bytes + p.w_bytes + p.sa_bytes + p.sb_bytes;
+  return p.x_bytes + p.w_bytes + p.sa_bytes + p.sb_bytes + p.part_bytes;
 }
 
 int mxk_linear_i8(const void* x_packed, int64_t x_nbytes, const float* x_scales, int64_t x_nscales, int64_t x_block,
@@ -1641,6 +1650,9 @@ int mxk_linear_i8(const void* x_packed, int64_t x_nbytes, const float* x_scales,
   const int8_t* B8 = p.direct_w ? (const int8_t*)w_packed : reinterpret_cast<int8_t*>(ws + p.x_bytes);
   float* sa = reinterpret_cast<float*>(ws + p.x_bytes + p.w_bytes);
   float* sb = reinterpret_cast<float*>(ws + p.x_bytes + p.w_bytes + p.sa_bytes);
+  if (p.mid.taken && reinterpret_cast<uintptr_t>(x_packed) % 4 == 0 && reinterpret_cast<uintptr_t>(w_packed) % 4 == 0)
+    return run_mid_lin(p.mid, x_packed, x_scales, x_block, w_packed, w_scales, w_block, M, K, N, x_bits, p.kblk, bias,
+                       out, workspace_nbytes >= need + p.part_bytes ? reinterpret_cast<float*>(ws + need) : nullptr, st);
   const int cap = num_cus() * 8;
   if (!p.direct_x) {
     const int64_t total = p.Mpad * (K / 16);

@@ -1,7 +1,9 @@
 // Packed block-scaled GEMM of middle sizes for gfx950 (mxk_gemm.hip states the
 // arithmetic): int8 or int4 operands as stored, blocks of 128 or 64, any M, K
 // and N.  It runs the shapes that the 256x128 loop does not take: grids below
-// one such tile per CU, blocks of 64, rows that do not start on 16 bytes.
+// one such tile per CU, blocks of 64, rows that do not start on 16 bytes.  BT
+// is the linear's form: [N][K] weights (B goes to LDS like A), scales by two
+// strides, and K in gridDim.y parts where the tiles alone leave CUs idle.
 //
 // A workgroup owns a 128x128 tile (8 waves of 32x64) or a 64x64 tile (4 waves
 // of 32x32).  A stage is 128 codes of K: one block of 128 or two of 64.  Its
@@ -35,15 +37,16 @@ struct MidArgs {
   const uint8_t* A;  // [M][K] codes
   const uint8_t* B;  // [K][N] codes, or (BT) [N][K]
   const float* sa;   // of row m, block kb: sa[m * sa_m + kb * sa_k]
-  const float* sb;   // of column n: sb[kb * N + n]
+  const float* sb;   // of column n: sb[kb * N + n], or (BT) sb[n * sb_n + kb * sb_k]
   float* C;          // fp32 C, or null
   int32_t* acc;      // [KB][M][N] integer products, or null
   uint8_t* cq;       // REQ: packed codes and scales of C
   float* cq_scales;
   const float* bias; // added to C when written (or null)
-  int64_t sa_m, sa_k;
+  int64_t sa_m, sa_k, sb_n, sb_k;
   uint32_t a_bytes, b_bytes, sa_bytes, sb_bytes;
   int M, K, N, KB, a_ok, b_ok, tiles_n, tiles;
+  int per;           // (BT) stages per K split: split z of gridDim.y writes C + z * M * N
 };
 
 constexpr uint32_t MID_OOB = 0x80000000u;
@@ -114,7 +117,8 @@ __global__ __launch_bounds__(TM * 4, TM == 128 ? 2 : 3) void k_qgemm_mid(MidArgs
   const __amdgpu_buffer_rsrc_t rA = make_rsrc(g.A, g.a_bytes), rB = make_rsrc(g.B, g.b_bytes);
   const __amdgpu_buffer_rsrc_t rSA = make_rsrc(g.sa, g.sa_bytes), rSB = make_rsrc(g.sb, g.sb_bytes);
 
-  const int stages = (g.K + 127) / 128;
+  const int st0 = BT ? (int)blockIdx.y * g.per : 0;
+  const int stages = BT ? std::min((g.K + 127) / 128, st0 + g.per) : (g.K + 127) / 128;
   // this thread's pieces: code index at stage 0, and what a stage adds
   uint32_t fa[Q], fb[Q];
   bool oka[Q], okb[Q];
@@ -156,8 +160,8 @@ __global__ __launch_bounds__(TM * 4, TM == 128 ? 2 : 3) void k_qgemm_mid(MidArgs
     }
     const int kb = st * H + sh_h;
     const bool ok = s_ok && kb < g.KB && !s_one;
-    const uint32_t off = ok ? (uint32_t)(s_a ? (m0 + sx) * g.sa_m + kb * g.sa_k : (int64_t)kb * g.N + n0 + sx - TM) * 4u
-                            : MID_OOB;
+    const int64_t so = BT ? (n0 + sx - TM) * g.sb_n + kb * g.sb_k : (int64_t)kb * g.N + n0 + sx - TM;
+    const uint32_t off = ok ? (uint32_t)(s_a ? (m0 + sx) * g.sa_m + kb * g.sa_k : so) * 4u : MID_OOB;
     // (two loads, one of them past its buffer: the resource is the wave's)
     const uint32_t va = buf_load_b32(rSA, s_a ? off : MID_OOB, 0u), vb = buf_load_b32(rSB, s_a ? MID_OOB : off, 0u);
     S.s = s_ok && kb < g.KB ? (s_one ? 1.0f : __uint_as_float(va | vb)) : 0.0f;
@@ -212,16 +216,16 @@ __global__ __launch_bounds__(TM * 4, TM == 128 ? 2 : 3) void k_qgemm_mid(MidArgs
   // one stage on its way in registers, two in LDS (stages past the last read
   // zeros); a second one in registers measured no faster
   Set S;
-  load(S, 0);
-  put(S, 0, 0);
-  load(S, 1);
+  load(S, st0);
+  put(S, st0, 0);
+  load(S, st0 + 1);
   if constexpr (NBUF > 2) {
-    put(S, 1, 1);
-    load(S, 2);
+    put(S, st0 + 1, 1);
+    load(S, st0 + 2);
   }
   __syncthreads();
-  for (int st = 0; st < stages; ++st) {
-    const int buf = st & (NBUF - 1);
+  for (int st = st0; st < stages; ++st) {
+    const int buf = (st - st0) & (NBUF - 1);
     const uint8_t* sA = lds + buf * STAGE;
     const uint8_t* sB = lds + NBUF * STAGE + buf * STAGE;
     const float* sS = reinterpret_cast<const float*>(lds + 2 * NBUF * STAGE) + buf * SC;
@@ -250,7 +254,7 @@ __global__ __launch_bounds__(TM * 4, TM == 128 ? 2 : 3) void k_qgemm_mid(MidArgs
       }
     // the readers of that buffer passed the last barrier
     constexpr int AHEAD = NBUF / 2;
-    put(S, st + AHEAD, (st + AHEAD) & (NBUF - 1));
+    put(S, st + AHEAD, (st - st0 + AHEAD) & (NBUF - 1));
     load(S, st + AHEAD + 1);
 #pragma unroll
     for (int hb = 0; hb < H; ++hb) {
@@ -283,11 +287,12 @@ __global__ __launch_bounds__(TM * 4, TM == 128 ? 2 : 3) void k_qgemm_mid(MidArgs
         }
       }
     }
-    if (NBUF == 2 || (st & 1)) __syncthreads();
+    if (NBUF == 2 || ((st - st0) & 1)) __syncthreads();
   }
   if constexpr (NBUF > 2) __syncthreads();
 
   if (g.C) {
+    float* C = BT ? g.C + (int64_t)blockIdx.y * g.M * g.N : g.C;
 #pragma unroll
     for (int a = 0; a < RT; ++a)
 #pragma unroll
@@ -297,7 +302,7 @@ __global__ __launch_bounds__(TM * 4, TM == 128 ? 2 : 3) void k_qgemm_mid(MidArgs
 #pragma unroll
         for (int t = 0; t < CT; ++t) {
           const int col = n0 + wn * 16 * CT + 16 * t + lcol;
-          if (col < g.N) g.C[(int64_t)row * g.N + col] = g.bias ? c[a][t][i] + g.bias[col] : c[a][t][i];
+          if (col < g.N) C[(int64_t)row * g.N + col] = g.bias ? c[a][t][i] + g.bias[col] : c[a][t][i];
         }
       }
   }
@@ -416,6 +421,8 @@ int run_mid(const MidPlan& p, const void* a, const float* sa, int a_ok, const vo
   g.sb = sb;
   g.C = C;
   g.acc = acc;
+  g.sb_n = g.sb_k = 0;
+  g.per = 0;
   g.cq = (uint8_t*)cq;
   g.cq_scales = cq_scales;
   g.bias = nullptr;
@@ -437,6 +444,92 @@ int run_mid(const MidPlan& p, const void* a, const float* sa, int a_ok, const vo
   else if (block == 128) mid_launch<4, 128>(g, p.tm, req, shift, st);
   else mid_launch<4, 64>(g, p.tm, req, shift, st);
   return check_launch("qgemm");
+}
+
+// C = the sum of S partial products in order (+ bias)
+__global__ __launch_bounds__(256) void k_mid_reduce(const float* __restrict__ part, int S, int64_t n, int64_t N,
+                                                    const float* __restrict__ bias, float* __restrict__ C) {
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+    float v = part[i];
+    for (int z = 1; z < S; ++z) v += part[z * n + i];
+    C[i] = bias ? v + bias[i % N] : v;
+  }
+}
+
+// Which int8 x int8 linears (us, scales per token of x and per block of w;
+// 128 x 128 kernels and their passes | 64-tiles | 256 x 128 loop):
+//   8x512x512          12.1 |  5.8           8x4096x4096        51.0 | 11.0
+//   64x4096x4096       53.9 | 14.1           128x8192x1024      96.3 | 15.0
+//   512x2048x2048      32.0 | 17.8           1000x4096x4096     60.9 | 53.2
+//   300x4160x4000       199 | 34.9  (blocks of 64)
+//   2001x4160x4096      393 |  127  (blocks of 64)
+//   8x4096x32768          - | 33.6 | 46.5    1100x4096x4096     62.3 |    - | 49.4
+//   1500x4096x4096     64.0 | 83.4 | 52.2    3500x4096x2048     64.3 | 81.6 | 55.3
+//   int4: 8x4096x4096   134 | 11.2           1000x4096x4096      152 | 53.3
+//   int4: 1500x4096x4096 161 | 76.5 | 146   2000x4096x4096      163 | 98.3
+// The 64-tiles read scales and codes as they are stored, one launch.  They
+// take up to four tiles per CU (int4, which the 256 x 128 loop unpacks first:
+// eight) and, in blocks of 64, which that loop does not have, all sizes.  A
+// grid of fewer tiles than the CUs hold at once (three each) splits K into
+// parts of at least six stages; 8x4096x4096 unsplit 23.1 -> 11.0, in 16 parts
+// 13.0; 128x8192x1024 43.5 -> 15.0.
+MidLin plan_mid_lin(int64_t M, int64_t K, int64_t N, int bits, int64_t x_block, int64_t w_block, int kblk) {
+  MidLin p;
+  const int64_t lim = int64_t(1) << 31, KB = K / kblk;
+  if ((bits != 4 && bits != 8) || (x_block != kblk && x_block != K) || (w_block != kblk && w_block != K)) return p;
+  if ((M + 128) * (K + 256) >= lim || (K + 256) * (N + 128) >= lim || KB * (M + 128) * 4 >= lim ||
+      KB * (N + 128) * 4 >= lim)
+    return p;
+  const int64_t stages = ceil_div(K, 128), tiles = ceil_div(M, 64) * ceil_div(N, 64);
+  if (kblk == 128 && tiles > (bits == 8 ? 4 : 8) * (int64_t)num_cus()) return p;
+  p.taken = true;
+  const int64_t S = std::max<int64_t>(1, std::min<int64_t>(3 * num_cus() / tiles, stages / 6));
+  p.per = (int)ceil_div(stages, S);
+  p.splits = (int)ceil_div(stages, p.per);
+  return p;
+}
+
+int run_mid_lin(const MidLin& p, const void* x, const float* sx, int64_t x_block, const void* w, const float* sw,
+                int64_t w_block, int64_t M, int64_t K, int64_t N, int bits, int kblk, const float* bias, float* out,
+                float* part, hipStream_t st) {
+  const int64_t KB = K / kblk;
+  MidArgs g{};
+  const bool split = p.splits > 1 && part;
+  g.A = (const uint8_t*)x;
+  g.B = (const uint8_t*)w;
+  g.sa = sx;
+  g.sb = sw;
+  g.C = split ? part : out;
+  g.bias = split ? nullptr : bias;
+  g.sa_m = x_block == K ? 1 : KB;
+  g.sa_k = x_block == K ? 0 : 1;
+  g.sb_n = w_block == K ? 1 : KB;
+  g.sb_k = w_block == K ? 0 : 1;
+  g.a_bytes = (uint32_t)(M * K * bits / 8);
+  g.b_bytes = (uint32_t)(K * N * bits / 8);
+  g.sa_bytes = (uint32_t)(g.sa_m * M * 4);
+  g.sb_bytes = (uint32_t)(g.sb_n * N * 4);
+  g.M = (int)M;
+  g.K = (int)K;
+  g.N = (int)N;
+  g.KB = (int)KB;
+  g.a_ok = g.b_ok = 1;
+  g.tiles_n = (int)ceil_div(N, 64);
+  g.tiles = (int)(ceil_div(M, 64) * g.tiles_n);
+  g.per = split ? p.per : (int)ceil_div(K, 128);
+  const dim3 grid((unsigned)(8 * ceil_div(g.tiles, 8)), split ? (unsigned)p.splits : 1u), wg(256);
+  if (bits == 8 && kblk == 128)
+    hipLaunchKernelGGL((k_qgemm_mid<8, 128, 64, false, true, 0, false>), grid, wg, 0, st, g);
+  else if (bits == 8)
+    hipLaunchKernelGGL((k_qgemm_mid<8, 64, 64, false, true, 0, false>), grid, wg, 0, st, g);
+  else if (kblk == 128)
+    hipLaunchKernelGGL((k_qgemm_mid<4, 128, 64, false, true, 0, false>), grid, wg, 0, st, g);
+  else
+    hipLaunchKernelGGL((k_qgemm_mid<4, 64, 64, false, true, 0, false>), grid, wg, 0, st, g);
+  if (split)
+    hipLaunchKernelGGL(k_mid_reduce, dim3((unsigned)std::min<int64_t>(ceil_div(M * N, 256), 8 * num_cus())), dim3(256),
+                       0, st, part, p.splits, M * N, N, bias, out);
+  return check_launch("linear_i8");
 }
 
 }  // namespace mxk

@@ -680,6 +680,16 @@ MidPlan plan_mid(int64_t M, int64_t K, int64_t N, int bits, int block, int out_b
 int run_mid(const MidPlan& p, const void* a, const float* sa, int a_ok, const void* b, const float* sb, int b_ok,
             int64_t M, int64_t K, int64_t N, int bits, int block, bool req, void* cq, float* cq_scales, float* C,
             int32_t* acc, hipStream_t st);
+// the same kernel with [N][K] weights and, for few tiles, K split over part
+// [splits][M][N] (part null: no split)
+struct MidLin {
+  bool taken = false;
+  int splits = 1, per = 0;  // K splits, stages of 128 in each
+};
+MidLin plan_mid_lin(int64_t M, int64_t K, int64_t N, int bits, int64_t x_block, int64_t w_block, int kblk);
+int run_mid_lin(const MidLin& p, const void* x, const float* sx, int64_t x_block, const void* w, const float* sw,
+                int64_t w_block, int64_t M, int64_t K, int64_t N, int bits, int kblk, const float* bias, float* out,
+                float* part, hipStream_t st);
 
 // Hadamard rotation of rows of 129 .. 8192 elements (mxk_rot.hip): to fp32, or
 // fused with the quantizer / decoder of blocks of 128 (MXK_EUNSUPPORTED with
