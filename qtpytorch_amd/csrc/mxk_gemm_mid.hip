@@ -36,8 +36,8 @@ typedef int32_t i2v __attribute__((ext_vector_type(2)));
 struct MidArgs {
   const uint8_t* A;  // [M][K] codes
   const uint8_t* B;  // [K][N] codes, or (BT) [N][K]
-  const float* sa;   // of row m, block kb: sa[m * sa_m + kb * sa_k]
-  const float* sb;   // of column n: sb[kb * N + n], or (BT) sb[n * sb_n + kb * sb_k]
+  const float* sa;   // of row m, block kb: sa[m * sa_m + kb * sa_k], or (BT) that index >> sa_sh
+  const float* sb;   // of column n: sb[kb * N + n], or (BT) sb[(n * sb_n + kb * sb_k) >> sb_sh]
   float* C;          // fp32 C, or null
   int32_t* acc;      // [KB][M][N] integer products, or null
   uint8_t* cq;       // REQ: packed codes and scales of C
@@ -46,6 +46,7 @@ struct MidArgs {
   int64_t sa_m, sa_k, sb_n, sb_k;
   uint32_t a_bytes, b_bytes, sa_bytes, sb_bytes;
   int M, K, N, KB, a_ok, b_ok, tiles_n, tiles;
+  int sa_sh, sb_sh;
   int per;           // (BT) stages per K split: split z of gridDim.y writes C + z * M * N
 };
 
@@ -160,8 +161,10 @@ __global__ __launch_bounds__(TM * 4, TM == 128 ? 2 : 3) void k_qgemm_mid(MidArgs
     }
     const int kb = st * H + sh_h;
     const bool ok = s_ok && kb < g.KB && !s_one;
-    const int64_t so = BT ? (n0 + sx - TM) * g.sb_n + kb * g.sb_k : (int64_t)kb * g.N + n0 + sx - TM;
-    const uint32_t off = ok ? (uint32_t)(s_a ? (m0 + sx) * g.sa_m + kb * g.sa_k : so) * 4u : MID_OOB;
+    const int64_t sa_i = (m0 + sx) * g.sa_m + kb * g.sa_k;
+    const int64_t sb_i = BT ? (n0 + sx - TM) * g.sb_n + kb * g.sb_k : (int64_t)kb * g.N + n0 + sx - TM;
+    const uint32_t off = ok ? (uint32_t)(BT ? (s_a ? sa_i >> g.sa_sh : sb_i >> g.sb_sh) : (s_a ? sa_i : sb_i)) * 4u
+                            : MID_OOB;
     // (two loads, one of them past its buffer: the resource is the wave's)
     const uint32_t va = buf_load_b32(rSA, s_a ? off : MID_OOB, 0u), vb = buf_load_b32(rSB, s_a ? MID_OOB : off, 0u);
     S.s = s_ok && kb < g.KB ? (s_one ? 1.0f : __uint_as_float(va | vb)) : 0.0f;
@@ -422,6 +425,7 @@ int run_mid(const MidPlan& p, const void* a, const float* sa, int a_ok, const vo
   g.C = C;
   g.acc = acc;
   g.sb_n = g.sb_k = 0;
+  g.sa_sh = g.sb_sh = 0;
   g.per = 0;
   g.cq = (uint8_t*)cq;
   g.cq_scales = cq_scales;
@@ -456,6 +460,14 @@ __global__ __launch_bounds__(256) void k_mid_reduce(const float* __restrict__ pa
   }
 }
 
+// One scale per row, or per power of two of the kernel's K blocks (block 128
+// on rows of odd multiples of 64: a scale may reach over two rows;
+// 9x5056x6968 with x's quantization 243 -> 31 us)
+static bool mid_scale_form(int64_t block, int64_t K, int kblk) {
+  const int64_t r = block / kblk;
+  return block == K || (r & (r - 1)) == 0;
+}
+
 // Which int8 x int8 linears (us, scales per token of x and per block of w;
 // 128 x 128 kernels and their passes | 64-tiles | 256 x 128 loop):
 //   8x512x512          12.1 |  5.8           8x4096x4096        51.0 | 11.0
@@ -476,7 +488,7 @@ __global__ __launch_bounds__(256) void k_mid_reduce(const float* __restrict__ pa
 MidLin plan_mid_lin(int64_t M, int64_t K, int64_t N, int bits, int64_t x_block, int64_t w_block, int kblk) {
   MidLin p;
   const int64_t lim = int64_t(1) << 31, KB = K / kblk;
-  if ((bits != 4 && bits != 8) || (x_block != kblk && x_block != K) || (w_block != kblk && w_block != K)) return p;
+  if ((bits != 4 && bits != 8) || !mid_scale_form(x_block, K, kblk) || !mid_scale_form(w_block, K, kblk)) return p;
   if ((M + 128) * (K + 256) >= lim || (K + 256) * (N + 128) >= lim || KB * (M + 128) * 4 >= lim ||
       KB * (N + 128) * 4 >= lim)
     return p;
@@ -505,10 +517,12 @@ int run_mid_lin(const MidLin& p, const void* x, const float* sx, int64_t x_block
   g.sa_k = x_block == K ? 0 : 1;
   g.sb_n = w_block == K ? 1 : KB;
   g.sb_k = w_block == K ? 0 : 1;
+  g.sa_sh = x_block == K ? 0 : __builtin_ctzll((uint64_t)(x_block / kblk));
+  g.sb_sh = w_block == K ? 0 : __builtin_ctzll((uint64_t)(w_block / kblk));
   g.a_bytes = (uint32_t)(M * K * bits / 8);
   g.b_bytes = (uint32_t)(K * N * bits / 8);
-  g.sa_bytes = (uint32_t)(g.sa_m * M * 4);
-  g.sb_bytes = (uint32_t)(g.sb_n * N * 4);
+  g.sa_bytes = (uint32_t)(ceil_div(M * K, x_block) * 4);
+  g.sb_bytes = (uint32_t)(ceil_div(N * K, w_block) * 4);
   g.M = (int)M;
   g.K = (int)K;
   g.N = (int)N;

@@ -58,7 +58,9 @@ def test_large(M, N, wd, wb, xb):
     (8, 768, 512, "int8d", 768, 128), (8, 1536, 70, "int8d", 1536, 128), (17, 3264, 200, "int8d", 64, 64),
     (64, 4096, 256, "int4d", 4096, 4096), (63, 1792, 129, "int4d", 128, 128), (129, 320, 2000, "int8d", 320, 64),
     (40, 512, 96, "int8d", 256, 128), (40, 512, 96, "int8d", 1024, 128), (1100, 1024, 4096, "int8d", 1024, 128),
-    (2049, 128, 4000, "int4d", 128, 128), (1090, 192, 4100, "int8d", 192, 64)])
+    (2049, 128, 4000, "int4d", 128, 128), (1090, 192, 4100, "int8d", 192, 64),
+    (57, 704, 816, "int8d", 704, 128), (33, 192, 70, "int4d", 128, 256), (9, 320, 129, "int8d", 128, 1024),
+    (9, 384, 129, "int8d", 128, 384), (9, 384, 129, "int8d", 768, 1152)])
 def test_tiles(M, K, N, dt, xb, wb):
     _check(M, K, N, dt, dt, xb, wb, bias=M % 2 == 1)
 
