@@ -164,10 +164,11 @@ __host__ __device__ __forceinline__ int64_t lm_xoff(int64_t m, int64_t k, int64_
 __host__ __device__ __forceinline__ int64_t lm_rows16(int64_t M) { return (M + 15) & ~(int64_t)15; }
 
 // ---------------------------------------------------------------- prepasses
-// Row m of x: ex[m] such that its largest |x| times 2^ex lies in [1, 2)
-// (0 for a zero row), and x * 2^ex zero-padded to Kp columns, as fp32
-// (SPLIT false) or as f16 hi + lo (SPLIT true: hi = RN16(v), lo = RN16(v - hi),
-// v - hi exact in fp32).  VEC: 16-byte rows (K * sizeof(T) % 16 == 0, x
+// Row m of x: ex[m] such that its largest |x| times 2^ex lies in [2^TOP,
+// 2^(TOP + 1)) (0 for a zero row), and x * 2^ex zero-padded to Kp columns, as
+// fp32 (SPLIT false) or as f16 hi + lo (SPLIT true: hi = RN16(v), lo = RN16(v -
+// hi), v - hi exact in fp32; a value keeps 2^-25, so 2^(-25 - TOP) of its row's
+// largest).  VEC: 16-byte rows (K * sizeof(T) % 16 == 0, x
 // 16-byte aligned); rows of up to 2048 16-byte chunks stay in registers
 // between the maximum and the scaled copy, longer ones are read twice.
 // LO false (16-bit x only) leaves lo out: an fp16 or bf16 value times a
@@ -195,7 +196,7 @@ __device__ __forceinline__ int64_t lm_prep_m(int64_t b, int64_t M) {
 }
 
 // Row m by one workgroup of 256 threads (red: 4 floats of LDS)
-template <typename T, bool SPLIT, bool VEC, bool LO = true>
+template <typename T, bool SPLIT, int TOP, bool VEC, bool LO = true>
 __device__ __forceinline__ void lm_prep_row(const T* __restrict__ x, int64_t m, int64_t K, int64_t Kp,
                                             float* __restrict__ xs, _Float16* __restrict__ xh,
                                             _Float16* __restrict__ xl, int* __restrict__ ex, float* red) {
@@ -233,7 +234,7 @@ __device__ __forceinline__ void lm_prep_row(const T* __restrict__ x, int64_t m, 
   __syncthreads();
   mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
   const int be = (int)((__float_as_uint(mx) >> 23) & 0xFFu);
-  const int e = (be == 0xFF || mx == 0.0f) ? 0 : 127 - (be == 0 ? 1 : be);
+  const int e = (be == 0xFF || mx == 0.0f) ? 0 : 127 + TOP - (be == 0 ? 1 : be);
   if (tid == 0) ex[m] = e;
   if (cached) {
 #pragma unroll
@@ -307,7 +308,7 @@ __global__ __launch_bounds__(256) void k_linear_mfma_prep_rows(const T* __restri
     }
     return;
   }
-  lm_prep_row<T, SPLIT, VEC, LO>(x, lm_prep_m(blockIdx.x, M), K, Kp, xs, xh, xl, ex, red);
+  lm_prep_row<T, SPLIT, 0, VEC, LO>(x, lm_prep_m(blockIdx.x, M), K, Kp, xs, xh, xl, ex, red);
 }
 
 inline size_t lm_round(size_t v) { return (v + 255) & ~(size_t)255; }

@@ -30,9 +30,13 @@
 // SIMDs that hold two of the 393 tiles are 2/3 busy with VALU); 1.2e-6 off the
 // 64-bit product there, 3.1e-7 here.
 //
-// Range as in mxk_linear_mfma.hip: rows of x scaled to [1, 2) by 2^ex[m]; the
-// weight by 2^es, one per 128-column tile ([K][N]) or per column ([N][K]),
-// that keeps the largest |c s| at most 2^15.  An output that comes out as
+// Range.  Both operands are scaled by powers of two to just below f16's largest
+// values: rows of x by 2^ex[m], to [2^14, 2^15); the weight by 2^es, one per
+// 128-column tile ([K][N]) or per column ([N][K]), that keeps the largest |c s|
+// at most 2^15.  An f16 pair keeps 2^-25, so a value keeps 2^-39 of the largest
+// of its row: with rows at [1, 2) x kept 2^-25 of it, and outputs whose terms are
+// of x large where the weight is small were off by 4e-3 (3e-7 here).  Products
+// are at most 2^30 and their sums below 2^55.  An output that comes out as
 // NaN (infinities or NaN in x or in the scales; inf - inf in a split) is
 // computed again as a plain fp32 sum, so that infinities come out as the
 // scalar kernel gives them.
@@ -451,7 +455,7 @@ __global__ __launch_bounds__(256) void k_linear_ragged_prep(const T* __restrict_
   __shared__ float sm[32];
   const int tid = threadIdx.x, lane = tid & 63;
   if ((int64_t)blockIdx.x < a.M) {
-    lm_prep_row<T, true, VEC, LO>(x, lm_prep_m(blockIdx.x, a.M), a.K, a.Kp, nullptr, xh, xl, ex, sm);
+    lm_prep_row<T, true, 14, VEC, LO>(x, lm_prep_m(blockIdx.x, a.M), a.K, a.Kp, nullptr, xh, xl, ex, sm);
     return;
   }
   const int64_t b = (int64_t)blockIdx.x - a.M;

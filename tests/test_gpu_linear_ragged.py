@@ -4,9 +4,11 @@ no multiple of 128, or blocks other than 128.
 
 Checked against x.double() @ dequant(W).double() with the oracle's dequantized
 weight.  The kernel carries x and c * s as f16 pairs hi + lo and leaves out lo
-* lo: each term is off by at most 3 * 2^-22 of itself, the fp32 sums add at
-most one rounding of 2^-24 per 32 terms and partial, and a value far below
-its row's (column tile's) largest keeps 2^-25 of that largest."""
+* lo: each term is off by at most 3 * 2^-22 of itself, and the fp32 sums add at
+most one rounding of 2^-24 per 32 terms and partial.  Rows of x and columns of W
+(of [in, out] weights: groups of 8 columns, which may meet one block) are scaled
+by powers of two that put their largest value at 2^13 or more, where f16 keeps
+2^-25: a value far below that largest is off by 2^-38 of it."""
 import pytest
 import torch
 
@@ -44,9 +46,12 @@ def _run(qa, x, packed, scales, dt, K, N, block, nt, bias=None):
 def _check(y, x, wd, nt, bias=None):
     xd, w = x.double(), (wd.t() if nt else wd).double()
     ref = xd @ w + (0 if bias is None else bias.double())
-    K = x.shape[1]
+    K, N = w.shape
     terms = xd.abs() @ w.abs()
-    floor = xd.abs().amax(1, keepdim=True) * w.abs().sum(0) * 2.0 ** -24
+    wmax = w.abs().amax(0)
+    if not nt:
+        wmax = torch.nn.functional.pad(wmax, (0, -N % 8)).view(-1, 8).amax(1).repeat_interleave(8)[:N]
+    floor = 2.0 ** -38 * (xd.abs().amax(1, keepdim=True) * w.abs().sum(0) + xd.abs().sum(1, keepdim=True) * wmax)
     tol = (3 * 2.0 ** -22 + (K / 32 + 16) * 2.0 ** -24) * terms + floor + 2.0 ** -23 * ref.abs() + 1e-37
     err = (y.double() - ref).abs()
     assert bool((err <= tol).all()), f"worst {float((err / tol).max()):.3g} x the bound"
@@ -81,7 +86,7 @@ def test_blocks(qa, block, nt):
 
 @pytest.mark.parametrize("nt", [False, True], ids=["kn", "nk"])
 def test_magnitudes(qa, nt):
-    """Rows of x and blocks of W of very different magnitudes, and a zero row."""
+    """Rows of x of very different magnitudes, a zero row, and small and large W."""
     M, K, N = 40, 513, 321
     x, _, _, _ = _case(M, K, N, "int8d", 128, nt, torch.float32)
     x *= 10.0 ** torch.linspace(-7, 7, M)[:, None]
@@ -93,6 +98,21 @@ def test_magnitudes(qa, nt):
         y = _run(qa, x, p, s, "int8d", K, N, 128, nt)
         _check(y, x, wd, nt)
         assert not y[3].any()
+
+
+@pytest.mark.parametrize("nt", [False, True], ids=["kn", "nk"])
+@pytest.mark.parametrize("M,src", [(8, torch.float32), (70, torch.float32), (70, torch.bfloat16)])
+@pytest.mark.parametrize("dt", FMTS)
+def test_mixed_k_magnitudes(qa, dt, M, src, nt):
+    """x large where W is small along K and the other way round: every term counts."""
+    K, N = (1000, 77) if nt else (2048, 203)
+    x, _, _, _ = _case(M, K, N, dt, 8, nt, src)
+    w = 0.02 * torch.randn(*((N, K) if nt else (K, N)), generator=torch.Generator().manual_seed(7))
+    small = torch.arange(K) // 8 % 2 == 0
+    x = torch.where(small, x.float() * 1e5, x.float()).to(src)
+    w *= torch.where(small, 1e-5, 1.0)[None, :] if nt else torch.where(small, 1e-5, 1.0)[:, None]
+    p, s, n = orc.quantize(w, dt, 8 if nt else 128)
+    _check(_run(qa, x, p, s, dt, K, N, 8 if nt else 128, nt), x, orc.dequant(p, s, dt, n, 8 if nt else 128).reshape(w.shape), nt)
 
 
 @pytest.mark.parametrize("nt", [False, True], ids=["kn", "nk"])
