@@ -35,7 +35,7 @@
 // 128-column tile ([K][N]) or per column ([N][K]), that keeps the largest |c s|
 // at most 2^15.  An f16 pair keeps 2^-25, so a value keeps 2^-39 of the largest
 // of its row: with rows at [1, 2) x kept 2^-25 of it, and outputs whose terms are
-// of x large where the weight is small were off by 4e-3 (3e-7 here).  Products
+// of x large where the weight is small were off by 4e-3 (4e-7 here).  Products
 // are at most 2^30 and their sums below 2^55.  An output that comes out as
 // NaN (infinities or NaN in x or in the scales; inf - inf in a split) is
 // computed again as a plain fp32 sum, so that infinities come out as the
@@ -293,6 +293,23 @@ __global__ __launch_bounds__(RG_WAVES * 64, 2) void k_linear_ragged(RgArgs a) {
       f += ldw;
     }
   };
+  // The step that K ends in: places past K hold the next column's ([N][K]) or the
+  // padding's codes, whose scales this column's exponent may take past f16's
+  // range, and x's zero times infinity is NaN.  Their scales become zeros.  A
+  // block that begins before K's end is this column's own.
+  const int kcut = (a.K & 31) != 0 ? a.steps - 1 : -1;
+  auto cut = [&](Step& p) {
+    const int left = (int)(a.K - 32 * (int64_t)kcut) - 8 * g;  // rows of this lane before K's end
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const bool gone = WT ? left <= 0 : i >= left;
+      p.sa[i] = gone ? 0.0f : p.sa[i];
+      if constexpr (STR) {
+        const bool past = gone || (WT && left < 8 && p.pre[i] >= (1u << left) - 1u);
+        p.sb[i] = past ? 0.0f : p.sb[i];
+      }
+    }
+  };
   auto tiles = [&](const Step& p, const XA& x) {
     auto scale = [&](int i, const int u) __attribute__((always_inline)) -> float {  // of code u of group i
       if constexpr (!STR) return p.sa[i];
@@ -369,6 +386,7 @@ __global__ __launch_bounds__(RG_WAVES * 64, 2) void k_linear_ragged(RgArgs a) {
         const int cur = st + p * WK, nx = cur + DR * WK;  // a step past s1 computes on zeros
         Step sp;
         take(sp, r[p % DR], cur);
+        if (cur == kcut) cut(sp);
         load_raw(r[p % DR], nx, nx < s1);
         if constexpr (DX == 2 && DR == 1) load_x(x[p ^ 1], nx, nx < s1);
         __builtin_amdgcn_sched_barrier(0);

@@ -117,6 +117,29 @@ def test_mixed_k_magnitudes(qa, dt, M, src, nt):
 
 @pytest.mark.parametrize("nt", [False, True], ids=["kn", "nk"])
 @pytest.mark.parametrize("M", [3, 70])
+@pytest.mark.parametrize("dt", FMTS)
+def test_columns_do_not_see_what_lies_past_k(qa, dt, M, nt):
+    """K no multiple of a step: the last step also loads the next row of an [out,
+    in] weight, or the padding of the last block.  A column keeps its bits when
+    the scales there grow by 2^20 (a rescued NaN would be another sum)."""
+    for K, N, block in (((1000, 40, 8), (1001, 60, 8), (133, 200, 128), (4100, 24, 128)) if nt
+                        else ((1001, 391, 128), (4100, 203, 64))):
+        x, p, s, _ = _case(M, K, N, dt, block, nt, torch.float32)
+        q = torch.arange(s.numel()) * block
+        if nt:  # blocks inside the odd rows
+            loud = (q // K % 2 == 1) & ((q + block - 1) // K == q // K)
+            keep = torch.arange(N) % 2 == 0
+        else:  # the last block; the tiles before it
+            loud = torch.arange(s.numel()) == s.numel() - 1
+            keep = torch.arange(N) < (int(q[-1]) - (K - 1) * N) // 128 * 128
+        assert loud.any() and keep.any()
+        a = _run(qa, x, p, s, dt, K, N, block, nt)
+        b = _run(qa, x, p, torch.where(loud, s * 2.0 ** 20, s), dt, K, N, block, nt)
+        assert torch.equal(a[:, keep], b[:, keep]), (K, N, block)
+
+
+@pytest.mark.parametrize("nt", [False, True], ids=["kn", "nk"])
+@pytest.mark.parametrize("M", [3, 70])
 def test_non_finite(qa, nt, M):
     """Infinities and NaN in x and in the scales come out where an fp32 product has them."""
     K, N = 300, 203
