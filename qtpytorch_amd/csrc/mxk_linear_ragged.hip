@@ -32,9 +32,12 @@
 //
 // Range.  Both operands are scaled by powers of two to just below f16's largest
 // values: rows of x by 2^ex[m], to [2^14, 2^15); the weight by 2^es, one per
-// 128-column tile ([K][N]) or per column ([N][K]), that keeps the largest |c s|
-// at most 2^15.  An f16 pair keeps 2^-25, so a value keeps 2^-39 of the largest
-// of its row: with rows at [1, 2) x kept 2^-25 of it, and outputs whose terms are
+// column ([N][K]) or per group of columns ([K][N]: of 8 for blocks below 128, of
+// 32 from there on, whose columns share three blocks in four), that keeps the
+// largest |c s| at most 2^15.  Scales that are not
+// finite are left out of es: they spoil their own columns alone.  An f16 pair
+// keeps 2^-25, so a value keeps 2^-38 of the largest of its row or columns (with
+// one es per 128 columns, a column lost bits beside others 2^16 times larger): with rows at [1, 2) x kept 2^-25 of it, and outputs whose terms are
 // of x large where the weight is small were off by 4e-3 (4e-7 here).  Products
 // are at most 2^30 and their sums below 2^55.  An output that comes out as
 // NaN (infinities or NaN in x or in the scales; inf - inf in a split) is
@@ -50,14 +53,14 @@ namespace mxk {
 namespace {
 
 constexpr int RG_WAVES = 4;
-constexpr int RG_CHUNKS = 8;  // parts of K that the largest scale of a column tile is found in
+constexpr int RG_CHUNKS = 8;  // parts of K that the largest scale of a group of columns is found in
 
 struct RgArgs {
   const void* x;       // the caller's x (recomputed outputs)
   const _Float16* xh;  // hi and lo of x * 2^ex, tiled (lm_xoff)
   const _Float16* xl;
   const int* ex;       // [M]
-  const float* smax;   // largest |scale|: [RG_CHUNKS][column tiles] or, WT, [N]
+  const float* smax;   // largest finite |scale|: [RG_CHUNKS][groups of 2^gsh columns of all tiles] or, WT, [N]
   const uint8_t* w;
   const float* scales;
   const float* bias;
@@ -67,6 +70,7 @@ struct RgArgs {
   uint32_t wbytes, sbytes, block, sh;  // block = 2^sh
   int M, x_type, wm, steps, sps, S;
   int tiles, per_xcd, mtiles;  // column tiles, those of one XCD, row groups
+  int gsh;                     // ([K][N]) groups of 2^gsh columns share an exponent
 };
 
 // Largest |c s| 2^es is at most 2^15: s 2^es below 2^(15 - bits of the largest |c|)
@@ -74,16 +78,22 @@ __host__ __device__ constexpr int rg_scale_top(int fmt) {
   return fmt == LM_I8 ? 8 : fmt == LM_I4 ? 12 : fmt == LM_I2 ? 14 : fmt == LM_I1 ? 15 : fmt == LM_F8 ? 14 : 26;
 }
 
-// The exponent that brings the scales of column n to their range (0 for a zero or non-finite maximum)
+// The exponent that brings the scales of column n to their range (0 for a zero maximum)
 template <int FMT, bool WT>
 __device__ __forceinline__ int rg_exponent(const RgArgs& a, int64_t n) {
-  float mx = a.smax[WT ? n : n / 128];
+  float mx = a.smax[WT ? n : n >> a.gsh];
   if constexpr (!WT) {
 #pragma unroll
-    for (int c = 1; c < RG_CHUNKS; ++c) mx = fmaxf(mx, a.smax[c * a.tiles + n / 128]);
+    for (int c = 1; c < RG_CHUNKS; ++c) mx = fmaxf(mx, a.smax[c * ((128 * a.tiles) >> a.gsh) + (n >> a.gsh)]);
   }
   const int be = (int)((__float_as_uint(mx) >> 23) & 0xFFu);
-  return (be == 0xFF || mx == 0.0f) ? 0 : rg_scale_top(FMT) + 126 - (be == 0 ? 1 : be);
+  return mx == 0.0f ? 0 : rg_scale_top(FMT) + 126 - (be == 0 ? 1 : be);
+}
+
+// The bits of |s|, 0 for infinities and NaN
+__device__ __forceinline__ uint32_t rg_finite(float s) {
+  const uint32_t b = mag_bits(s);
+  return b < 0x7F800000u ? b : 0u;
 }
 
 // The packed codes of a lane's 8 x 8 block as loaded, and its scales
@@ -207,7 +217,7 @@ __global__ __launch_bounds__(RG_WAVES * 64, 2) void k_linear_ragged(RgArgs a) {
   int esv[8];
 #pragma unroll
   for (int t = 0; t < 8; ++t)
-    esv[t] = rg_exponent<FMT, WT>(a, WT ? min((int64_t)nl + t, a.N - 1) : (int64_t)n0);
+    esv[t] = rg_exponent<FMT, WT>(a, WT ? min((int64_t)nl + t, a.N - 1) : (int64_t)nl);
 
   // flat index of group i (row 8g + i, or column 8j + i) of a step
   auto flat0 = [&](int step) -> uint32_t {
@@ -462,52 +472,84 @@ __global__ __launch_bounds__(256) void k_linear_ragged_reduce(RgArgs a) {
 }
 
 // Workgroups 0 .. M - 1: a row of x each (lm_prep_row); the others the largest
-// |scale|: of four columns each ([N][K], one wave per column), or of 8 column
-// tiles over one of RG_CHUNKS parts of K each ([K][N]; 8 threads side by side
-// read the scales of 8 tiles, which lie together: with one tile per workgroup
-// every lane met a line of its own, 15 us at 4096 x 50257).
+// finite |scale|: of four columns each ([N][K], one wave per column), or of the
+// groups of columns of 8 column tiles over one of RG_CHUNKS parts of K each
+// ([K][N]; 8 threads side by side read the scales of 8 tiles, which lie together:
+// with one tile per workgroup every lane met a line of its own, 15 us at 4096 x
+// 50257).  Blocks of 128 and more: at most two meet a row of a tile, and the
+// groups of 32 are kept in registers (groups of 8 in LDS: 7.7 us there).
 template <typename T, bool VEC, bool WT, bool LO>
 __global__ __launch_bounds__(256) void k_linear_ragged_prep(const T* __restrict__ x, RgArgs a, _Float16* __restrict__ xh,
                                                             _Float16* __restrict__ xl, int* __restrict__ ex,
                                                             float* __restrict__ smax) {
-  __shared__ float sm[32];
+  __shared__ float sm[4];
   const int tid = threadIdx.x, lane = tid & 63;
   if ((int64_t)blockIdx.x < a.M) {
     lm_prep_row<T, true, 14, VEC, LO>(x, lm_prep_m(blockIdx.x, a.M), a.K, a.Kp, nullptr, xh, xl, ex, sm);
     return;
   }
   const int64_t b = (int64_t)blockIdx.x - a.M;
-  float mx = 0.0f;
   if constexpr (WT) {
     const int64_t n = 4 * b + (tid >> 6);
     if (n >= a.N) return;
+    float mx = 0.0f;
     const uint32_t q0 = (uint32_t)((n * a.K) >> a.sh), q1 = (uint32_t)((n * a.K + a.K - 1) >> a.sh);
-    for (uint32_t q = q0 + lane; q <= q1; q += 64) mx = fmaxf(mx, __builtin_fabsf(a.scales[q]));
+    for (uint32_t q = q0 + lane; q <= q1; q += 64) mx = fmaxf(mx, __uint_as_float(rg_finite(a.scales[q])));
     mx = group_max<64>(mx);
     if (lane == 0) smax[n] = mx;
   } else {
-    const uint32_t tile = (uint32_t)(b / RG_CHUNKS) * 8u + (tid & 7), ch = (uint32_t)(b % RG_CHUNKS);
-    const uint32_t N = (uint32_t)a.N, K = (uint32_t)a.K, per = (K + RG_CHUNKS - 1) / RG_CHUNKS;
-    const uint32_t k1 = min(K, (ch + 1) * per);
-    if (tile < (uint32_t)a.tiles) {
-      const uint32_t n0 = 128u * tile, n1 = min(n0 + 128u, N) - 1u;
-      if (a.sh >= 7) {  // blocks of 128 and more: at most two meet a row of the tile
-#pragma unroll 8
-        for (uint32_t k = ch * per + (tid >> 3); k < k1; k += 32)
-          mx = fmaxf(mx, fmaxf(__builtin_fabsf(a.scales[(k * N + n0) >> a.sh]),
-                               __builtin_fabsf(a.scales[(k * N + n1) >> a.sh])));
-      } else {
-        for (uint32_t k = ch * per + (tid >> 3); k < k1; k += 32)
-          for (uint32_t q = (k * N + n0) >> a.sh; q <= (k * N + n1) >> a.sh; ++q)
-            mx = fmaxf(mx, __builtin_fabsf(a.scales[q]));
-      }
-    }
+    __shared__ uint32_t gm[128];  // [wave][tile][4 groups of 32], or [tile][16 of 8]
+    const uint32_t tile0 = (uint32_t)(b / RG_CHUNKS) * 8u, tile = tile0 + (tid & 7), ch = (uint32_t)(b % RG_CHUNKS);
+    const uint32_t N = (uint32_t)a.N, K = (uint32_t)a.K, tiles = (uint32_t)a.tiles, per = (K + RG_CHUNKS - 1) / RG_CHUNKS;
+    const uint32_t k1 = min(K, (ch + 1) * per), n0 = 128u * tile, cl = min(128u, N - n0) - 1u;  // (cl: its last column)
+    if (a.gsh == 5) {
+      uint32_t m[4] = {0u, 0u, 0u, 0u};
+      if (tile < tiles) {
+        // the loads of 8 rows at a time (past the last row: that row again)
+        for (uint32_t k = ch * per + (tid >> 3); k < k1; k += 256) {
+          uint32_t c[8];
+          float s0[8], s1[8];
 #pragma unroll
-    for (int o = 8; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-    if (lane < 8) sm[(tid >> 6) * 8 + lane] = mx;
-    __syncthreads();
-    if (tid < 8 && tile < (uint32_t)a.tiles)
-      smax[ch * (uint32_t)a.tiles + tile] = fmaxf(fmaxf(sm[tid], sm[8 + tid]), fmaxf(sm[16 + tid], sm[24 + tid]));
+          for (int u = 0; u < 8; ++u) {
+            const uint32_t f = min(k + 32u * u, k1 - 1u) * N + n0, q = f >> a.sh;
+            c[u] = ((q + 1u) << a.sh) - f;  // the second block's column
+            s0[u] = a.scales[q];
+            s1[u] = a.scales[(f + cl) >> a.sh];
+          }
+#pragma unroll
+          for (int u = 0; u < 8; ++u) {
+            const uint32_t v0 = rg_finite(s0[u]), v1 = rg_finite(s1[u]);
+#pragma unroll
+            for (uint32_t w = 0; w < 4; ++w) m[w] = max(m[w], max(32u * w < c[u] ? v0 : 0u, 32u * w + 32u > c[u] ? v1 : 0u));
+          }
+        }
+      }
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+#pragma unroll
+        for (int o = 8; o < 64; o <<= 1) m[w] = max(m[w], (uint32_t)__shfl_xor((int)m[w], o));
+        if (lane < 8) gm[(tid >> 6) * 32 + 4 * lane + w] = m[w];
+      }
+      __syncthreads();
+      if (tid < 32 && tile0 + tid / 4 < tiles)
+        smax[ch * 4u * tiles + 4u * tile0 + tid] =
+            __uint_as_float(max(max(gm[tid], gm[32 + tid]), max(gm[64 + tid], gm[96 + tid])));
+    } else {
+      if (tid < 128) gm[tid] = 0u;
+      __syncthreads();
+      if (tile < tiles) {
+        for (uint32_t k = ch * per + (tid >> 3); k < k1; k += 32) {
+          const uint32_t f = k * N + n0;
+          for (uint32_t q = f >> a.sh; q <= (f + cl) >> a.sh; ++q) {
+            const uint32_t c0 = max(q << a.sh, f) - f, c1 = min((q << a.sh) + a.block - 1u - f, cl);
+            const uint32_t v = rg_finite(a.scales[q]);
+            for (uint32_t c = c0 >> 3; c <= c1 >> 3; ++c) atomicMax(&gm[16 * (tid & 7) + c], v);
+          }
+        }
+      }
+      __syncthreads();
+      if (tid < 128 && tile0 + tid / 16 < tiles) smax[ch * 16u * tiles + 16u * tile0 + tid] = __uint_as_float(gm[tid]);
+    }
   }
 }
 
@@ -556,7 +598,7 @@ RgPlan rg_plan(int64_t M, int64_t K, int64_t N) {
   p.off_ex = o;
   o += lm_round((size_t)M * 4);
   p.off_es = o;
-  o += lm_round((size_t)N * 4);
+  o += lm_round((size_t)ceil_div(N, 128) * 128 * 4);  // N, or RG_CHUNKS times at most 16 groups per tile
   p.off_x = o;
   o += lm_round((size_t)lm_rows16(M) * (size_t)p.Kp * 4);
   p.off_p = o;
@@ -654,6 +696,7 @@ int rg_run(const void* x, int x_type, int64_t M, int64_t K, const void* w, int64
   a.sps = p.sps;
   a.S = p.S;
   a.tiles = (int)ceil_div(N, 128);
+  a.gsh = l >= 7 ? 5 : 3;
   a.per_xcd = (int)ceil_div(a.tiles, 8);
   a.mtiles = (int)ceil_div(M, 16 * p.rt * p.wm);
   if (x_type == MXK_IN_F32) rg_prep<WT, float>(p, a, xh, xl, ex, smax, st);

@@ -6,9 +6,10 @@ Checked against x.double() @ dequant(W).double() with the oracle's dequantized
 weight.  The kernel carries x and c * s as f16 pairs hi + lo and leaves out lo
 * lo: each term is off by at most 3 * 2^-22 of itself, and the fp32 sums add at
 most one rounding of 2^-24 per 32 terms and partial.  Rows of x and columns of W
-(of [in, out] weights: groups of 8 columns, which may meet one block) are scaled
-by powers of two that put their largest value at 2^13 or more, where f16 keeps
-2^-25: a value far below that largest is off by 2^-38 of it."""
+(of [in, out] weights: groups of 8 columns, or of 32 in blocks of 128 and more)
+are scaled by powers of two that put their largest value at 2^13 or more, where f16 keeps
+2^-25: a value far below that largest is off by 2^-38 of it (of weights: of the
+largest value that the blocks of its columns can hold)."""
 import pytest
 import torch
 
@@ -43,14 +44,16 @@ def _run(qa, x, packed, scales, dt, K, N, block, nt, bias=None):
     return fn(x.to(d), packed.to(d), scales.to(d), dt, *sizes, block, bias=None if bias is None else bias.to(d)).cpu()
 
 
-def _check(y, x, wd, nt, bias=None):
+def _check(y, x, wd, nt, bias=None, top=None, block=128):
+    """top: the largest value each weight's block can hold (else |wd|)."""
     xd, w = x.double(), (wd.t() if nt else wd).double()
     ref = xd @ w + (0 if bias is None else bias.double())
     K, N = w.shape
     terms = xd.abs() @ w.abs()
-    wmax = w.abs().amax(0)
+    wmax = (w.abs() if top is None else top.t() if nt else top).double().amax(0)
     if not nt:
-        wmax = torch.nn.functional.pad(wmax, (0, -N % 8)).view(-1, 8).amax(1).repeat_interleave(8)[:N]
+        g = 32 if block >= 128 else 8
+        wmax = torch.nn.functional.pad(wmax, (0, -N % g)).view(-1, g).amax(1).repeat_interleave(g)[:N]
     floor = 2.0 ** -38 * (xd.abs().amax(1, keepdim=True) * w.abs().sum(0) + xd.abs().sum(1, keepdim=True) * wmax)
     tol = (3 * 2.0 ** -22 + (K / 32 + 16) * 2.0 ** -24) * terms + floor + 2.0 ** -23 * ref.abs() + 1e-37
     err = (y.double() - ref).abs()
@@ -81,7 +84,7 @@ def test_blocks(qa, block, nt):
     for dt in ("int4d", "int8d", "float8d"):
         for M, K, N in ((4, 160, 256), (70, 133, 77)):
             x, p, s, wd = _case(M, K, N, dt, block, nt, torch.float32)
-            _check(_run(qa, x, p, s, dt, K, N, block, nt), x, wd, nt)
+            _check(_run(qa, x, p, s, dt, K, N, block, nt), x, wd, nt, block=block)
 
 
 @pytest.mark.parametrize("nt", [False, True], ids=["kn", "nk"])
@@ -136,6 +139,35 @@ def test_columns_do_not_see_what_lies_past_k(qa, dt, M, nt):
         a = _run(qa, x, p, s, dt, K, N, block, nt)
         b = _run(qa, x, p, torch.where(loud, s * 2.0 ** 20, s), dt, K, N, block, nt)
         assert torch.equal(a[:, keep], b[:, keep]), (K, N, block)
+
+
+@pytest.mark.parametrize("nt", [False, True], ids=["kn", "nk"])
+@pytest.mark.parametrize("M", [3, 70])
+@pytest.mark.parametrize("dt", FMTS)
+def test_column_magnitudes(qa, dt, M, nt):
+    """Columns far smaller than the ones beside them, and one scale that is not
+    finite: every other column keeps its own precision."""
+    for block, K, N in ((8, 300, 264), (8, 77, 131), (64, 333, 391), (128, 600, 203), (256, 1025, 300), (128, 4100, 140)):
+        if nt:
+            K, N = N, K
+        x, p, s, _ = _case(M, K, N, dt, block, nt, torch.float32)
+        g = torch.Generator().manual_seed(K)
+        flat = torch.arange(s.numel()) * block
+        # a magnitude for each row of [out, in] weights, for each place of a block's start of [in, out] ones
+        mag = torch.exp2(-30 * torch.rand(N, generator=g))
+        s = s * (mag[flat // K] if nt else mag[(flat % N) // 16 * 16])
+        q = 5 if nt else s.numel() // 2
+        s[q] = (float("inf"), float("nan"))[M % 2]
+        wd = orc.dequant(p, s, dt, K * N, block).reshape((N, K) if nt else (K, N))
+        y = _run(qa, x, p, s, dt, K, N, block, nt)
+        vmax = 1.0 if dt[0] == "f" or dt == "int1d" else float(2 ** (int(dt[3]) - 1) - 1)
+        top = (vmax * torch.where(s.isfinite(), s, 0.0)).repeat_interleave(block)[:K * N].reshape(wd.shape)
+        ok = wd.isfinite().all(1 if nt else 0)
+        assert 0 < int(ok.sum()) < N
+        assert not y[:, ~ok].isfinite().any()
+        # (groups of columns keep their place: what is left out counts as zero)
+        wd = torch.where(ok[:, None] if nt else ok[None, :], wd, 0.0)
+        _check(torch.where(ok[None, :], y, 0.0), x, wd, nt, top=top, block=block)
 
 
 @pytest.mark.parametrize("nt", [False, True], ids=["kn", "nk"])
