@@ -164,6 +164,9 @@ __host__ __device__ __forceinline__ int64_t lm_xoff(int64_t m, int64_t k, int64_
 __host__ __device__ __forceinline__ int64_t lm_rows16(int64_t M) { return (M + 15) & ~(int64_t)15; }
 
 // ---------------------------------------------------------------- prepasses
+// ex[m] of a row that holds a NaN: all its outputs are NaN, whatever they are scaled by
+constexpr int LM_NAN_ROW = 1 << 20;
+
 // Row m of x: ex[m] such that its largest |x| times 2^ex lies in [2^TOP,
 // 2^(TOP + 1)) (0 for a zero row), and x * 2^ex zero-padded to Kp columns, as
 // fp32 (SPLIT false) or as f16 hi + lo (SPLIT true: hi = RN16(v), lo = RN16(v -
@@ -212,7 +215,7 @@ __device__ __forceinline__ void lm_prep_row(const T* __restrict__ x, int64_t m, 
 #pragma unroll
     for (int e = 0; e < E; ++e) v[e] = ElemT<T>::cvt(t[e]);
   };
-  float mx = 0.0f;
+  uint32_t mx = 0u;
   if (cached) {
 #pragma unroll
     for (int q = 0; q < NCH; ++q) {
@@ -224,18 +227,18 @@ __device__ __forceinline__ void lm_prep_row(const T* __restrict__ x, int64_t m, 
       float v[E];
       elems(c[q], v);
 #pragma unroll
-      for (int e = 0; e < E; ++e) mx = fmaxf(mx, __builtin_fabsf(v[e]));
+      for (int e = 0; e < E; ++e) mx = max(mx, mag_bits(v[e]));
     }
   } else {
-    for (int64_t k = tid; k < K; k += 256) mx = fmaxf(mx, __builtin_fabsf(ElemT<T>::cvt(row[k])));
+    for (int64_t k = tid; k < K; k += 256) mx = max(mx, mag_bits(ElemT<T>::cvt(row[k])));
   }
-  mx = group_max<64>(mx);
-  if ((tid & 63) == 0) red[tid >> 6] = mx;
+  mx = group_max_u<64>(mx);
+  if ((tid & 63) == 0) red[tid >> 6] = __uint_as_float(mx);
   __syncthreads();
-  mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-  const int be = (int)((__float_as_uint(mx) >> 23) & 0xFFu);
-  const int e = (be == 0xFF || mx == 0.0f) ? 0 : 127 + TOP - (be == 0 ? 1 : be);
-  if (tid == 0) ex[m] = e;
+  mx = max(max(__float_as_uint(red[0]), __float_as_uint(red[1])), max(__float_as_uint(red[2]), __float_as_uint(red[3])));
+  const int be = (int)(mx >> 23);
+  const int e = (be == 0xFF || mx == 0u) ? 0 : 127 + TOP - (be == 0 ? 1 : be);
+  if (tid == 0) ex[m] = mx > 0x7F800000u ? LM_NAN_ROW : e;
   if (cached) {
 #pragma unroll
     for (int q = 0; q < NCH; ++q) {

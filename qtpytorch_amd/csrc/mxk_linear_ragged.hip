@@ -34,15 +34,21 @@
 // values: rows of x by 2^ex[m], to [2^14, 2^15); the weight by 2^es, one per
 // column ([N][K]) or per group of columns ([K][N]: of 8 for blocks below 128, of
 // 32 from there on, whose columns share three blocks in four), that keeps the
-// largest |c s| at most 2^15.  Scales that are not
-// finite are left out of es: they spoil their own columns alone.  An f16 pair
-// keeps 2^-25, so a value keeps 2^-38 of the largest of its row or columns (with
-// one es per 128 columns, a column lost bits beside others 2^16 times larger): with rows at [1, 2) x kept 2^-25 of it, and outputs whose terms are
-// of x large where the weight is small were off by 4e-3 (4e-7 here).  Products
-// are at most 2^30 and their sums below 2^55.  An output that comes out as
-// NaN (infinities or NaN in x or in the scales; inf - inf in a split) is
-// computed again as a plain fp32 sum, so that infinities come out as the
-// scalar kernel gives them.
+// largest |c s| at most 2^15.  Scales that are not finite are left out of es:
+// they spoil their own columns alone.  An f16 pair keeps 2^-25, so a value keeps
+// 2^-38 of the largest of its row or columns.  With rows at [1, 2) x kept 2^-25
+// of it, and outputs whose terms are of x large where the weight is small were
+// off by 4e-3 (4e-7 here); with one es per 128 columns a column lost bits beside
+// others 2^16 times larger.  Products are at most 2^30, their sums below 2^55.
+//
+// Infinities and NaN.  Only they, in x or in the scales, bring out a NaN here (inf -
+// inf in a split, 0 * inf).  A NaN in a row of x is a NaN in all of its outputs.
+// Any other one is summed again in fp32, over the terms that are not finite, so
+// that infinities come out as the scalar kernel gives them: the wave looks for
+// such terms 64 k at a time, and a lane sums its 4 rows x 8 columns of a row tile
+// side by side until all are NaN.  64 x 2048 x 1001 int8, 107 us (scalar kernel
+// 368): with a NaN 104 us, with infinities in every third row 571 (each output
+// by one lane over all of K: 3.3 and 52 ms).
 #include "mxk_linear_mfma.h"
 
 #include <algorithm>
@@ -154,28 +160,53 @@ __device__ __forceinline__ uint32_t rg_pair_along(uint32_t w0, uint32_t w1, int 
   }
 }
 
-// One output as the plain fp32 sum of the scalar kernel (k ascending)
-template <int FMT, bool WT>
-__device__ __forceinline__ float rg_scalar(const RgArgs& a, int64_t m, int64_t n) {
+// The weight c * s at flat index `flat` and the element (m, k) of x, in fp32
+template <int FMT>
+__device__ __forceinline__ float rg_weight(const RgArgs& a, uint32_t flat) {
   constexpr int BITS = lm_bits(FMT);
-  float acc = 0.0f;
-  for (int64_t k = 0; k < a.K; ++k) {
-    const int64_t flat = WT ? n * a.K + k : k * a.N + n;
-    const uint32_t code = ((uint32_t)a.w[flat * BITS / 8] >> ((flat * BITS) & 7)) & ((1u << BITS) - 1u);
-    const float s = a.scales[flat / a.block];
-    float c;
-    if constexpr (FMT == LM_F8) {
-      c = (float)__builtin_bit_cast(h2v, lm_pair<FMT>(code << 8))[0] * lm_post(FMT);
-    } else {
-      c = (float)__builtin_bit_cast(h2v, lm_pair<FMT>(code))[0] * lm_post(FMT);
+  const uint32_t bit = (flat & 7u) * BITS;  // (flat * BITS may not fit 32 bits)
+  const uint32_t code = ((uint32_t)a.w[(flat >> 3) * BITS + (bit >> 3)] >> (bit & 7u)) & ((1u << BITS) - 1u);
+  const uint32_t pair = lm_pair<FMT>(FMT == LM_F8 ? code << 8 : code);
+  return (float)__builtin_bit_cast(h2v, pair)[0] * lm_post(FMT) * a.scales[flat >> a.sh];
+}
+__device__ __forceinline__ float rg_x(const RgArgs& a, int64_t m, int64_t k) {
+  const int64_t at = m * a.K + k;
+  return a.x_type == MXK_IN_F32   ? ((const float*)a.x)[at]
+         : a.x_type == MXK_IN_F16 ? ElemT<__half>::cvt(((const __half*)a.x)[at])
+                                  : ElemT<hip_bfloat16>::cvt(((const hip_bfloat16*)a.x)[at]);
+}
+
+// The places k0 .. k0 + 63 whose terms may not be finite in the row tile at mt
+// (rows that hold a NaN aside) and the column tile at n0, as a mask; the wave's
+// 64 lanes together
+template <bool WT>
+__device__ __forceinline__ uint64_t rg_odd(const RgArgs& a, int64_t mt, uint32_t n0, int64_t k0, int lane) {
+  const int64_t kl = min(k0 + lane, a.K - 1);
+  bool odd = false, all = false;
+  auto rows = [&](const auto* x, uint32_t emask) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int64_t m = min(mt + r, (int64_t)a.M - 1);
+      const uint32_t b = x[m * a.K + kl];
+      odd = odd || (a.ex[m] != LM_NAN_ROW && (b & emask) == emask);
     }
-    const float wv = c * s;
-    const float xv = a.x_type == MXK_IN_F32   ? ((const float*)a.x)[m * a.K + k]
-                     : a.x_type == MXK_IN_F16 ? ElemT<__half>::cvt(((const __half*)a.x)[m * a.K + k])
-                                              : ElemT<hip_bfloat16>::cvt(((const hip_bfloat16*)a.x)[m * a.K + k]);
-    acc = __builtin_fmaf(xv, wv, acc);
+  };
+  if (a.x_type == MXK_IN_F32) rows((const uint32_t*)a.x, 0x7F800000u);
+  else rows((const uint16_t*)a.x, a.x_type == MXK_IN_F16 ? 0x7C00u : 0x7F80u);
+  auto scales = [&](int64_t f0, int64_t f1) {
+    bool hit = false;
+    for (uint32_t q = (uint32_t)f0 >> a.sh; q <= (uint32_t)f1 >> a.sh; ++q)
+      hit = hit || mag_bits(a.scales[q]) >= 0x7F800000u;
+    return hit;
+  };
+  if constexpr (WT) {
+    for (int64_t n = (int64_t)n0 + lane; n < min((int64_t)n0 + 128, a.N); n += 64)
+      all = all || scales(n * a.K + k0, n * a.K + min(k0 + 63, a.K - 1));
+  } else {
+    odd = odd || scales(kl * a.N + n0, kl * a.N + min((int64_t)n0 + 127, a.N - 1));
   }
-  return acc;
+  const uint64_t in = a.K - k0 >= 64 ? ~0ull : (1ull << (a.K - k0)) - 1;
+  return (__ballot(all) != 0 ? ~0ull : __ballot(odd)) & in;
 }
 
 // the finished output from its sum in the scaled units
@@ -442,18 +473,53 @@ __global__ __launch_bounds__(RG_WAVES * 64, 2) void k_linear_ragged(RgArgs a) {
       for (int t = 0; t < 8; ++t) {
         if ((int64_t)nl + t >= a.N) continue;
         const float v = acc[i][t][q];
-        bad = bad || v != v;
+        bad = bad || (v != v && exm != LM_NAN_ROW);
         dst[t] = a.part ? v : rg_finish<FMT>(v, -(exm + esv[t])) + (a.bias ? a.bias[nl + t] : 0.0f);
       }
     }
-  // outputs that came out as NaN: again, in full (this lane wrote them)
-  if (a.part || !bad) return;
+  if (a.part || __ballot(bad) == 0) return;
 #pragma unroll 1
-  for (int e = 0; e < RT * 32; ++e) {
-    const int64_t m = m0 + 16 * (e >> 5) + 4 * g + ((e >> 3) & 3), n = (int64_t)nl + (e & 7);
-    if (m >= a.M || n >= a.N) continue;
-    const float v = a.out[m * a.N + n];
-    if (v != v) a.out[m * a.N + n] = rg_scalar<FMT, WT>(a, m, n) + (a.bias ? a.bias[n] : 0.0f);
+  for (int i = 0; i < RT; ++i) {
+    const int64_t mt = m0 + 16 * i, m = mt + 4 * g;
+    uint32_t todo = 0u;  // bit 8 q + t: the output of row m + q and column nl + t (which this lane wrote)
+    for (int e = 0; e < 32; ++e) {
+      const int64_t mr = m + (e >> 3), n = (int64_t)nl + (e & 7);
+      if (mr >= a.M || n >= a.N || a.ex[mr] == LM_NAN_ROW) continue;
+      const float v = a.out[mr * a.N + n];
+      todo |= (v != v ? 1u : 0u) << e;
+    }
+    if (__ballot(todo != 0u) == 0) continue;
+    float y[4][8];
+#pragma unroll
+    for (int e = 0; e < 32; ++e) y[e >> 3][e & 7] = 0.0f;
+    bool open = true;
+#pragma unroll 1
+    for (int64_t k0 = 0; k0 < a.K && open; k0 += 64) {
+      uint64_t odd = rg_odd<WT>(a, mt, n0, k0, lane);
+      while (odd != 0 && open) {
+        const int64_t k = k0 + __builtin_ctzll(odd);
+        odd &= odd - 1;
+        float xv[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) xv[q] = rg_x(a, min(m + q, (int64_t)a.M - 1), k);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+          const int64_t n = min((int64_t)nl + t, a.N - 1);
+          const float w = rg_weight<FMT>(a, (uint32_t)(WT ? n * a.K + k : k * a.N + n));
+#pragma unroll
+          for (int q = 0; q < 4; ++q) y[q][t] = __builtin_fmaf(xv[q], w, y[q][t]);
+        }
+        uint32_t nan = 0u;
+#pragma unroll
+        for (int e = 0; e < 32; ++e) nan |= (y[e >> 3][e & 7] != y[e >> 3][e & 7] ? 1u : 0u) << e;
+        open = __ballot((todo & ~nan) != 0u) != 0;
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 32; ++e) {
+      const int64_t n = (int64_t)nl + (e & 7);
+      if ((todo >> e) & 1u) a.out[(m + (e >> 3)) * a.N + n] = y[e >> 3][e & 7] + (a.bias ? a.bias[n] : 0.0f);
+    }
   }
 }
 
@@ -466,7 +532,12 @@ __global__ __launch_bounds__(256) void k_linear_ragged_reduce(RgArgs a) {
     for (int z = 1; z < a.S; ++z) v += a.part[z * total + i];
     const int64_t m = i / a.N, n = i - m * a.N;
     float y = rg_finish<FMT>(v, -(a.ex[m] + rg_exponent<FMT, WT>(a, n)));
-    if (v != v) y = rg_scalar<FMT, WT>(a, m, n);
+    if (v != v && a.ex[m] != LM_NAN_ROW) {
+      y = 0.0f;
+#pragma unroll 8
+      for (int64_t k = 0; k < a.K; ++k)
+        y = __builtin_fmaf(rg_x(a, m, k), rg_weight<FMT>(a, (uint32_t)(WT ? n * a.K + k : k * a.N + n)), y);
+    }
     a.out[i] = a.bias ? y + a.bias[n] : y;
   }
 }

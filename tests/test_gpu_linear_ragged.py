@@ -188,6 +188,73 @@ def test_non_finite(qa, nt, M):
     assert float(((y.double() - ref)[fin]).abs().max()) <= 1e-3 * float(ref[fin].abs().max())
 
 
+@pytest.mark.parametrize("nt", [False, True], ids=["kn", "nk"])
+@pytest.mark.parametrize("dt", FMTS)
+@pytest.mark.parametrize("M,K,N", [(6, 300, 203), (70, 301, 140), (20, 4100, 77)])
+def test_non_finite_rows_and_columns(qa, M, K, N, dt, nt):
+    """Whole rows and single values of NaN and of infinities of one and both
+    signs, beside a scale that is infinite and one that is NaN, with and without
+    K split: NaN, infinities and finite values where a 64-bit product has them."""
+    for src in (torch.float32, torch.bfloat16):
+        x, p, s, _ = _case(M, K, N, dt, 128, nt, src)
+        x[0, :], x[1, 7], x[2, 5], x[2, 6] = float("inf"), float("nan"), float("inf"), -float("inf")
+        x[3, :], x[4, K - 1] = float("nan"), -float("inf")
+        s[3], s[-1] = float("inf"), float("nan")
+        wd = orc.dequant(p, s, dt, K * N, 128).reshape((N, K) if nt else (K, N))
+        bias = torch.randn(N)
+        y = _run(qa, x, p, s, dt, K, N, 128, nt, bias)
+        # (one product after the other: a library's sum may meet its operands padded)
+        t = x.double()[:, :, None] * (wd.t() if nt else wd).double()[None]
+        ref = t.sum(1) + bias
+        assert torch.equal(y.isnan(), ref.isnan()) and torch.equal(y.isinf(), ref.isinf())
+        assert torch.equal(y[y.isinf()].sign().double(), ref[ref.isinf()].sign())
+        fin = ref.isfinite()
+        assert not fin.any() or float((y.double() - ref)[fin].abs().max()) <= 1e-5 * float(ref[fin].abs().max())
+
+
+@pytest.mark.parametrize("nt", [False, True], ids=["kn", "nk"])
+def test_non_finite_rows_take_no_longer_than_the_scalar_kernel(qa, nt):
+    """A NaN in x costs nothing, infinities at most a small multiple of the fp32
+    kernel that runs without a workspace (the sum of one output after the other
+    took 30 times the product for a single NaN)."""
+    M, K, N = 64, 2048, 1001
+    if nt:
+        K, N = N, K
+    x, p, s, _ = _case(M, K, N, "int8d", 128, nt, torch.float32)
+    x, p, s = x.cuda(), p.cuda(), s.cuda()
+    lib, L = qa._lib.lib(), qa._lib
+    out = torch.empty(M, N, device="cuda")
+
+    def scalar():
+        if nt:
+            return lib.mxk_linear_wq_nt(x.data_ptr(), 0, M, K, p.data_ptr(), p.numel() * p.element_size(), s.data_ptr(),
+                                        s.numel(), 0, N, 0, 8, 128, 0, out.data_ptr(), 0, 0, L.stream_of(x))
+        return lib.mxk_linear_wq(x.data_ptr(), 0, M, K, p.data_ptr(), s.data_ptr(), 0, N, 0, 8, 128, 0, out.data_ptr(),
+                                 0, 0, L.stream_of(x))
+
+    def us(fn):
+        best = float("inf")
+        for _ in range(5):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            fn()
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b) * 1e3)
+        return best
+
+    fn = qa.ops.linear_wq_nt if nt else qa.ops.linear_wq
+    call = lambda v: fn(v, p, s, "int8d", *((N, K) if nt else (K, N)), 128)
+    assert scalar() == 0
+    one, rows, inf = x.clone(), x.clone(), x.clone()
+    one[5, 9] = rows[::2, 3] = float("nan")
+    inf[::3, 4] = float("inf")
+    base, fp32 = us(lambda: call(x)), us(scalar)
+    t = [us(lambda: call(v)) for v in (one, rows, inf)]
+    print(f"{nt} finite {base:.0f} us, scalar kernel {fp32:.0f}; a NaN {t[0]:.0f}, NaN rows {t[1]:.0f}, infinities {t[2]:.0f}")
+    assert max(t[:2]) < 3 * base and t[2] < 8 * fp32
+
+
 def test_module_and_gradient(qa):
     """mx_linear with an odd width: forward, input gradient and a captured replay."""
     g = torch.Generator().manual_seed(3)
