@@ -201,6 +201,18 @@ def _zeroed_workspace(nbytes: int, device, stream: int) -> Optional[Tensor]:
     return ws
 
 
+def _linear_workspace(decode_bytes: int, M: int, K: int, N: int, bits: int, block: int, device, stream: int):
+    """(buffer, bytes) for a weight-only linear: the stream's kept workspace where
+    the kernels need its cleared counters; else, for weights that the ragged
+    kernel takes, a buffer of this call alone (x in f16 pairs and partial sums,
+    4 M K bytes and more: 0.4 GB for 2048 rows by 50257, which nobody would give
+    back)."""
+    if decode_bytes > 0:
+        return _zeroed_workspace(decode_bytes, device, stream), decode_bytes
+    nbytes = L.lib().mxk_linear_ragged_workspace(M, K, N, bits, block)
+    return (torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None), nbytes
+
+
 def quantize(x: Tensor, dt, block: int = 128, *, seed: Optional[int] = None,
              signs: Optional[Tensor] = None, n_store: Optional[int] = None
              ) -> Tuple[Tensor, Tensor, int]:
@@ -448,10 +460,9 @@ def linear_wq(x: Tensor, w_packed: Optional[Tensor], w_scales: Tensor, dt, in_fe
     if b is not None and b.data_ptr() % 16:
         b = b.clone()
     lib = L.lib()
-    ws_bytes = (lib.mxk_linear_workspace(M, K, N, dt.bits, block)
-                or lib.mxk_linear_ragged_workspace(M, K, N, dt.bits, block))
     stream = L.stream_of(xc)
-    ws = _zeroed_workspace(ws_bytes, dev, stream)
+    ws, ws_bytes = _linear_workspace(lib.mxk_linear_workspace(M, K, N, dt.bits, block), M, K, N, dt.bits, block, dev,
+                                     stream)
     with L.on_device(dev):
         rc = L.MXK_EUNSUPPORTED
         if w_tiled is not None and w_scales_t is not None and decode_prepack_eligible(dt, block, K, N):
@@ -651,10 +662,9 @@ def linear_wq_nt(x: Tensor, w_packed: Optional[Tensor], w_scales: Tensor, dt, ou
             raise L.MXKError("linear_wq_nt: w_tiled must be prepack_weight_nt() of this weight (uint8, "
                              "contiguous, same device)")
     lib = L.lib()
-    ws_bytes = (lib.mxk_linear_nt_workspace(M, K, N, dt.bits, block)
-                or lib.mxk_linear_ragged_workspace(M, K, N, dt.bits, block))
     stream = L.stream_of(xc)
-    wk = _zeroed_workspace(ws_bytes, dev, stream)
+    wk, ws_bytes = _linear_workspace(lib.mxk_linear_nt_workspace(M, K, N, dt.bits, block), M, K, N, dt.bits, block, dev,
+                                     stream)
     with L.on_device(dev):
         rc = L.MXK_EUNSUPPORTED
         if w_tiled is not None and w_scales_t is not None and decode_prepack_nt_eligible(dt, block, K, N):

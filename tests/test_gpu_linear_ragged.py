@@ -255,6 +255,26 @@ def test_non_finite_rows_take_no_longer_than_the_scalar_kernel(qa, nt):
     assert max(t[:2]) < 3 * base and t[2] < 8 * fp32
 
 
+@pytest.mark.parametrize("nt", [False, True], ids=["kn", "nk"])
+def test_keeps_no_workspace(qa, nt):
+    """A call's scratch memory (x again, and the partial sums) goes back with it."""
+    M, K, N = 16, 8192, 1001
+    if nt:
+        K, N = N, K
+    x, p, s, _ = _case(M, K, N, "int4d", 128, nt, torch.float32)
+    x, p, s = x.cuda(), p.cuda(), s.cuda()
+    fn = qa.ops.linear_wq_nt if nt else qa.ops.linear_wq
+    assert qa._lib.lib().mxk_linear_ragged_workspace(M, K, N, 4, 128) >= 4 * M * K
+    side = torch.cuda.Stream()  # a stream of its own: nothing kept for it yet
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        before = torch.cuda.memory_allocated()
+        y = fn(x, p, s, "int4d", *((N, K) if nt else (K, N)), 128)
+        held = torch.cuda.memory_allocated() - before
+    torch.cuda.current_stream().wait_stream(side)
+    assert held <= y.numel() * 4 + 512
+
+
 def test_module_and_gradient(qa):
     """mx_linear with an odd width: forward, input gradient and a captured replay."""
     g = torch.Generator().manual_seed(3)
