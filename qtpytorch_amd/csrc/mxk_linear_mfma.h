@@ -82,18 +82,42 @@ __host__ __device__ constexpr uint32_t lm_sel_f(int a, int b) {
   return FMT == LM_F8 ? lm_selh(a, b) : lm_sel(a, b);
 }
 
-// p = x * s as f16 hi + lo for two elements: hi = RN16(x*s), lo =
-// RN16(x*s - hi), each one v_fma_mix (fp32 product, f16 result), so
-// |x*s - hi - lo| <= 2^-22 |x*s| (less for values whose lo is subnormal:
-// at most 2^-25 absolute).
-__device__ __forceinline__ void lm_split2(float x0, float s0, float x1, float s1, uint32_t& hi, uint32_t& lo) {
-  uint32_t h, l;
-  asm("v_fma_mixlo_f16 %0, %1, %2, 0 op_sel_hi:[0,0,0]" : "=v"(h) : "v"(x0), "v"(s0));
-  asm("v_fma_mixhi_f16 %0, %1, %2, 0 op_sel_hi:[0,0,0]" : "+v"(h) : "v"(x1), "v"(s1));
-  asm("v_fma_mixlo_f16 %0, %1, %2, -%3 op_sel_hi:[0,0,1]" : "=v"(l) : "v"(x0), "v"(s0), "v"(h));
-  asm("v_fma_mixhi_f16 %0, %1, %2, -%3 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "+v"(l) : "v"(x1), "v"(s1), "v"(h));
-  hi = h;
-  lo = l;
+// p = c * s as f16 hi + lo for four elements: hi = RN16(c s), lo = RN16(c s -
+// hi), each one v_fma_mix (fp32 product, f16 result), so |c s - hi - lo| <= 2^-22
+// |c s| (less for values whose lo is subnormal: at most 2^-25 absolute).  c is
+// four floats (F32) or two f16 pairs, in c[0] and c[2].  One asm statement: an
+// instruction that writes the high half of a register may not be followed at once
+// by one that reads it, and the compiler, which may move single asm statements
+// about, does not see that they do.  (The two wait states before an MFMA:
+// lm_settle.)
+template <bool F32>
+__device__ __forceinline__ void lm_split4(const uint32_t (&c)[4], const float (&s)[4], uint32_t& h0, uint32_t& h1,
+                                          uint32_t& l0, uint32_t& l1) {
+  if constexpr (F32) {
+    asm("v_fma_mixlo_f16 %0, %4, %8, 0 op_sel_hi:[0,0,0]\n\t"
+        "v_fma_mixlo_f16 %1, %6, %10, 0 op_sel_hi:[0,0,0]\n\t"
+        "v_fma_mixhi_f16 %0, %5, %9, 0 op_sel_hi:[0,0,0]\n\t"
+        "v_fma_mixhi_f16 %1, %7, %11, 0 op_sel_hi:[0,0,0]\n\t"
+        "v_fma_mixlo_f16 %2, %4, %8, -%0 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %3, %6, %10, -%1 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %2, %5, %9, -%0 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %3, %7, %11, -%1 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "s_nop 0"
+        : "=&v"(h0), "=&v"(h1), "=&v"(l0), "=&v"(l1)
+        : "v"(c[0]), "v"(c[1]), "v"(c[2]), "v"(c[3]), "v"(s[0]), "v"(s[1]), "v"(s[2]), "v"(s[3]));
+  } else {
+    asm("v_fma_mixlo_f16 %0, %4, %6, 0 op_sel_hi:[1,0,0]\n\t"
+        "v_fma_mixlo_f16 %1, %5, %8, 0 op_sel_hi:[1,0,0]\n\t"
+        "v_fma_mixhi_f16 %0, %4, %7, 0 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\t"
+        "v_fma_mixhi_f16 %1, %5, %9, 0 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\t"
+        "v_fma_mixlo_f16 %2, %4, %6, -%0 op_sel_hi:[1,0,1]\n\t"
+        "v_fma_mixlo_f16 %3, %5, %8, -%1 op_sel_hi:[1,0,1]\n\t"
+        "v_fma_mixhi_f16 %2, %4, %7, -%0 op_sel:[1,0,1] op_sel_hi:[1,0,1]\n\t"
+        "v_fma_mixhi_f16 %3, %5, %9, -%1 op_sel:[1,0,1] op_sel_hi:[1,0,1]\n\t"
+        "s_nop 0"
+        : "=&v"(h0), "=&v"(h1), "=&v"(l0), "=&v"(l1)
+        : "v"(c[0]), "v"(c[2]), "v"(s[0]), "v"(s[1]), "v"(s[2]), "v"(s[3]));
+  }
 }
 
 // Two wait states between the asm instructions that wrote a and b and the

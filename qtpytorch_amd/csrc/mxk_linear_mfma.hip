@@ -453,15 +453,19 @@ __global__ __launch_bounds__(LM_THREADS, 1) void k_linear_mfma(
       } else {
         u4v hv, lv;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int e = 2 * q;
-          const float x0 = __uint_as_float(a.x[i][e >> 2][e & 3]), x1 = __uint_as_float(a.x[i][e >> 2][(e & 3) + 1]);
-          const float s0 = __builtin_ldexpf(__uint_as_float(a.s[e >> 2][e & 3]), es_nb);
-          const float s1 = __builtin_ldexpf(__uint_as_float(a.s[e >> 2][(e & 3) + 1]), es_nb);
-          uint32_t hh, ll;
-          lm_split2(x0, s0, x1, s1, hh, ll);
-          hv[q] = hh;
-          lv[q] = ll;
+        for (int q = 0; q < 4; q += 2) {
+          uint32_t x[4], h0, h1, l0, l1;
+          float s[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            x[e] = a.x[i][q >> 1][e];
+            s[e] = __builtin_ldexpf(__uint_as_float(a.s[q >> 1][e]), es_nb);
+          }
+          lm_split4<true>(x, s, h0, h1, l0, l1);
+          hv[q] = h0;
+          hv[q + 1] = h1;
+          lv[q] = l0;
+          lv[q + 1] = l1;
         }
         ahi[i] = __builtin_bit_cast(h8v, hv);
         alo[i] = __builtin_bit_cast(h8v, lv);

@@ -109,38 +109,6 @@ struct RgRaw {
   uint32_t s[8][2];
 };
 
-// hi and lo of c * s for four codes and their scales: hi = RN16(c s), lo =
-// RN16(c s - hi).  The codes are two f16 pairs (F32 false) or four floats.
-// Two pairs in turn: an instruction that writes half a register may not be
-// followed at once by one that reads it.
-template <bool F32>
-__device__ __forceinline__ void rg_split4(const uint32_t (&c)[4], const float (&s)[4], uint32_t& h0, uint32_t& h1,
-                                          uint32_t& l0, uint32_t& l1) {
-#define RG_MIX(OP, D, MOD, C, S, REST) asm(OP " %0, %1, %2, " REST : MOD(D) : "v"(C), "v"(S))
-#define RG_MIXL(OP, D, MOD, C, S, H, REST) asm(OP " %0, %1, %2, -%3 " REST : MOD(D) : "v"(C), "v"(S), "v"(H))
-  if constexpr (F32) {
-    RG_MIX("v_fma_mixlo_f16", h0, "=v", c[0], s[0], "0 op_sel_hi:[0,0,0]");
-    RG_MIX("v_fma_mixlo_f16", h1, "=v", c[2], s[2], "0 op_sel_hi:[0,0,0]");
-    RG_MIX("v_fma_mixhi_f16", h0, "+v", c[1], s[1], "0 op_sel_hi:[0,0,0]");
-    RG_MIX("v_fma_mixhi_f16", h1, "+v", c[3], s[3], "0 op_sel_hi:[0,0,0]");
-    RG_MIXL("v_fma_mixlo_f16", l0, "=v", c[0], s[0], h0, "op_sel_hi:[0,0,1]");
-    RG_MIXL("v_fma_mixlo_f16", l1, "=v", c[2], s[2], h1, "op_sel_hi:[0,0,1]");
-    RG_MIXL("v_fma_mixhi_f16", l0, "+v", c[1], s[1], h0, "op_sel:[0,0,1] op_sel_hi:[0,0,1]");
-    RG_MIXL("v_fma_mixhi_f16", l1, "+v", c[3], s[3], h1, "op_sel:[0,0,1] op_sel_hi:[0,0,1]");
-  } else {
-    RG_MIX("v_fma_mixlo_f16", h0, "=v", c[0], s[0], "0 op_sel_hi:[1,0,0]");
-    RG_MIX("v_fma_mixlo_f16", h1, "=v", c[2], s[2], "0 op_sel_hi:[1,0,0]");
-    RG_MIX("v_fma_mixhi_f16", h0, "+v", c[0], s[1], "0 op_sel:[1,0,0] op_sel_hi:[1,0,0]");
-    RG_MIX("v_fma_mixhi_f16", h1, "+v", c[2], s[3], "0 op_sel:[1,0,0] op_sel_hi:[1,0,0]");
-    RG_MIXL("v_fma_mixlo_f16", l0, "=v", c[0], s[0], h0, "op_sel_hi:[1,0,1]");
-    RG_MIXL("v_fma_mixlo_f16", l1, "=v", c[2], s[2], h1, "op_sel_hi:[1,0,1]");
-    RG_MIXL("v_fma_mixhi_f16", l0, "+v", c[0], s[1], h0, "op_sel:[1,0,1] op_sel_hi:[1,0,1]");
-    RG_MIXL("v_fma_mixhi_f16", l1, "+v", c[2], s[3], h1, "op_sel:[1,0,1] op_sel_hi:[1,0,1]");
-  }
-#undef RG_MIX
-#undef RG_MIXL
-}
-
 // Byte b of w as a signed code, in float
 __device__ __forceinline__ uint32_t rg_i8(uint32_t w, int b) { return __float_as_uint((float)(int8_t)(w >> (8 * b))); }
 
@@ -376,7 +344,7 @@ __global__ __launch_bounds__(RG_WAVES * 64, 2) void k_linear_ragged(RgArgs a) {
 #pragma unroll
           for (int u = 0; u < 4; ++u)
             c[u] = WT ? rg_i8(p.c.w[2 * t + (q >> 1)], u) : rg_i8(p.c.w[2 * (2 * q + u) + (t >> 2)], t & 3);
-          rg_split4<true>(c, s, h0, h1, l0, l1);
+          lm_split4<true>(c, s, h0, h1, l0, l1);
         } else {
           if constexpr (WT) {
             c[0] = rg_pair_along<FMT>(p.c.w[BITS == 8 ? 2 * t : t], p.c.w[BITS == 8 ? 2 * t + 1 : t], q);
@@ -386,7 +354,7 @@ __global__ __launch_bounds__(RG_WAVES * 64, 2) void k_linear_ragged(RgArgs a) {
             c[2] = d[q + 1];
           }
           c[1] = c[3] = 0u;
-          rg_split4<false>(c, s, h0, h1, l0, l1);
+          lm_split4<false>(c, s, h0, h1, l0, l1);
         }
         bh[q] = h0;
         bh[q + 1] = h1;
