@@ -188,6 +188,10 @@ __host__ __device__ __forceinline__ int64_t lm_xoff(int64_t m, int64_t k, int64_
 __host__ __device__ __forceinline__ int64_t lm_rows16(int64_t M) { return (M + 15) & ~(int64_t)15; }
 
 // ---------------------------------------------------------------- prepasses
+// Rows of x in f16 pairs have their largest value in [2^14, 2^15): the pair then
+// keeps 2^-39 of it (at [1, 2): 2^-25).  The products stay far below fp32's limit.
+constexpr int LM_X_TOP = 14;
+
 // ex[m] of a row that holds a NaN: all its outputs are NaN, whatever they are scaled by
 constexpr int LM_NAN_ROW = 1 << 20;
 
@@ -335,7 +339,7 @@ __global__ __launch_bounds__(256) void k_linear_mfma_prep_rows(const T* __restri
     }
     return;
   }
-  lm_prep_row<T, SPLIT, 0, VEC, LO>(x, lm_prep_m(blockIdx.x, M), K, Kp, xs, xh, xl, ex, red);
+  lm_prep_row<T, SPLIT, SPLIT ? LM_X_TOP : 0, VEC, LO>(x, lm_prep_m(blockIdx.x, M), K, Kp, xs, xh, xl, ex, red);
 }
 
 inline size_t lm_round(size_t v) { return (v + 255) & ~(size_t)255; }

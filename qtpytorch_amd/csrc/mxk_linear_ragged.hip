@@ -524,7 +524,7 @@ __global__ __launch_bounds__(256) void k_linear_ragged_prep(const T* __restrict_
   __shared__ float sm[4];
   const int tid = threadIdx.x, lane = tid & 63;
   if ((int64_t)blockIdx.x < a.M) {
-    lm_prep_row<T, true, 14, VEC, LO>(x, lm_prep_m(blockIdx.x, a.M), a.K, a.Kp, nullptr, xh, xl, ex, sm);
+    lm_prep_row<T, true, LM_X_TOP, VEC, LO>(x, lm_prep_m(blockIdx.x, a.M), a.K, a.Kp, nullptr, xh, xl, ex, sm);
     return;
   }
   const int64_t b = (int64_t)blockIdx.x - a.M;

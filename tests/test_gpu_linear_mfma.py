@@ -20,6 +20,7 @@ import torch
 
 from oracle import mx_oracle as orc
 from tests import _golden as G
+from tests.test_gpu_linear_ragged import _check as _check_terms
 
 pytestmark = pytest.mark.gpu
 
@@ -366,7 +367,8 @@ def test_mx_linear_rotated_and_vector_weights(qa, dt):
 def test_16_bit_x_is_its_own_hi(qa, dt, src, M):
     """[out, in] weights: fp16 and bf16 x take one product per term.  Their
     scaled values are their own f16 hi, so the result is the fp32 path's bits,
-    also for values far below a row's largest."""
+    also for values far below a row's largest, and within the bound of a 64-bit
+    product."""
     K, N = 384, 256
     x = _randn((M, K), 31 + M) * 10.0 ** torch.linspace(-4, 4, M)[:, None]
     x[:, ::7] *= 2.0 ** -13
@@ -375,4 +377,22 @@ def test_16_bit_x_is_its_own_hi(qa, dt, src, M):
     w = 0.02 * _randn((N, K), 5)
     q = qa.mx_tensor.quantize(w.to(dev()), dt, 128)
     args = (q._mx_packed, q._mx_scales, q._mx_dtype, N, K, 128)
-    assert torch.equal(qa.ops.linear_wq_nt(x.to(dev()), *args), qa.ops.linear_wq_nt(x.float().to(dev()), *args))
+    y = qa.ops.linear_wq_nt(x.to(dev()), *args)
+    assert torch.equal(y, qa.ops.linear_wq_nt(x.float().to(dev()), *args))
+    _check_terms(y.cpu(), x, q.dequantize().cpu(), True)
+
+
+@pytest.mark.parametrize("dt", FMTS)
+@pytest.mark.parametrize("src", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M", [3, 40, 300])
+def test_out_in_mixed_k_magnitudes(qa, dt, src, M):
+    """[out, in] weights, x large in the blocks of K where W is small and the other
+    way round: every term counts."""
+    K, N = 1024, 256
+    small = (torch.arange(K) // 128 % 2 == 0)[None, :]
+    x = torch.where(small, 1e5, 1.0) * _randn((M, K), 41 + M)
+    w = 0.02 * torch.where(small, 1e-5, 1.0) * _randn((N, K), 43)
+    x = x.to(src)
+    q = qa.mx_tensor.quantize(w.to(dev()), dt, 128)
+    y = qa.ops.linear_wq_nt(x.to(dev()), q._mx_packed, q._mx_scales, q._mx_dtype, N, K, 128)
+    _check_terms(y.cpu(), x, q.dequantize().cpu(), True)
