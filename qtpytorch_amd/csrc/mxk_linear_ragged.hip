@@ -23,12 +23,13 @@
 // scales and a position.  Waves that split K meet in LDS in a fixed order, K
 // splits across workgroups in a second kernel.
 //
-// What bounds it: few rows, the decode (about 450 VALU per 32 x 128 step of a
+// What bounds it: few rows, the decode (about 480 VALU per 32 x 128 step of a
 // wave) and the number of column tiles against CUs; many rows, decode and MFMA
 // in equal parts (a wave decodes its weights for 64 rows).  16 x 4096 x 50257
-// int8: 1149 us on the scalar kernel, here 104 us (98 + 5 for the prepass; the
-// SIMDs that hold two of the 393 tiles are 2/3 busy with VALU); 1.2e-6 off the
-// 64-bit product there, 3.1e-7 here.
+// int8: 1149 us on the scalar kernel, here 97.7 (the profiler gives the product
+// 99 and the prepass 6 us, each by itself); VALU instructions take 56% of the
+// SIMDs' time, 73% where a CU holds two of the 393 tiles, MFMAs 9%.  1.2e-6 off
+// the 64-bit product there, 3.0e-7 here.
 //
 // Range.  Both operands are scaled by powers of two to just below f16's largest
 // values: rows of x by 2^ex[m], to [2^14, 2^15); the weight by 2^es, one per

@@ -15,7 +15,8 @@
 // 4096 x 4096 bf16 the rotation and the quantizer behind it took 64.5 + 12.0
 // us, the decoder and the unrotation 15.4 + 68.7 us (the rotated copy in fp32
 // between them); one kernel each here: 20.1 and 21.9 us, against 8 and 15
-// us for the bytes alone.
+// us for the bytes alone.  VALU bounds both: 40 and 42 instructions per
+// element, which at 4 cycles a wave fill the SIMDs' time.
 //
 // LDS place of element i: i + 4 (i / 16) + 16 (i / 256): the strided reads of
 // a pass (lanes 2^k apart) and the 16-byte reads of the last one meet

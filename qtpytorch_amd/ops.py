@@ -210,7 +210,7 @@ def _linear_workspace(decode_bytes: int, M: int, K: int, N: int, bits: int, bloc
     if decode_bytes > 0:
         return _zeroed_workspace(decode_bytes, device, stream), decode_bytes
     nbytes = L.lib().mxk_linear_ragged_workspace(M, K, N, bits, block)
-    return (torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None), nbytes
+    return _workspace(nbytes, device), nbytes
 
 
 def quantize(x: Tensor, dt, block: int = 128, *, seed: Optional[int] = None,
