@@ -19,31 +19,37 @@ typedef uint32_t u2v __attribute__((ext_vector_type(2)));
 constexpr uint32_t LM_OOB = 0x80000000u;       // past every buffer: loads return zeros
 constexpr size_t LM_WS_BASE = 65536;           // workspace bytes left to the decode kernels' counters
 
-// Two int4 codes at bits 0-3 and 16-19 of d (other bits ignored) as an f16
-// pair: 0x6400 | (c ^ 8) is the f16 1024 + (c + 8), exact, less 1032.
+// Integer codes as f16 pairs of c 2^-E (E 0 or 14): all values are exact and
+// normal, and E only changes constants.  The f16 2^(10 - E) with code bits in its
+// low bits is (1024 + code) 2^-E.
+template <int E>
+__device__ __forceinline__ uint32_t lm_ipair(uint32_t d, uint32_t flip, float bias) {
+  const uint32_t e = d ^ (((0x6400u - ((uint32_t)E << 10)) | flip) * 0x00010001u);
+  const _Float16 b = (_Float16)((1024.0f + bias) / (float)(1 << E));
+  return __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2v, e) - h2v{b, b});
+}
+// Two int4 codes at bits 0-3 and 16-19 of d (other bits ignored): c ^ 8 is c + 8
+template <int E = 0>
 __device__ __forceinline__ uint32_t lm_i4pair(uint32_t d) {
-  const uint32_t e = (d & 0x000F000Fu) ^ 0x64086408u;
-  const h2v r = __builtin_bit_cast(h2v, e) - h2v{(_Float16)1032.0f, (_Float16)1032.0f};
-  return __builtin_bit_cast(uint32_t, r);
+  return lm_ipair<E>(d & 0x000F000Fu, 8u, 8.0f);
 }
-// Two int8 codes at bits 0-7 and 16-23 of d (bits 8-15, 24-31 zero):
-// 0x6400 | (c ^ 0x80) is 1024 + (c + 128), less 1152.
+// Two int8 codes at bits 0-7 and 16-23 of d (bits 8-15, 24-31 zero)
+template <int E = 0>
 __device__ __forceinline__ uint32_t lm_i8pair(uint32_t d) {
-  const uint32_t e = d ^ 0x64806480u;
-  const h2v r = __builtin_bit_cast(h2v, e) - h2v{(_Float16)1152.0f, (_Float16)1152.0f};
-  return __builtin_bit_cast(uint32_t, r);
+  return lm_ipair<E>(d, 0x80u, 128.0f);
 }
-// Two int2 codes at bits 0-1 and 16-17 of d (other bits ignored):
-// 0x6400 | (c ^ 2) is 1024 + (c + 2), less 1026.
+// Two int2 codes at bits 0-1 and 16-17 of d (other bits ignored)
+template <int E = 0>
 __device__ __forceinline__ uint32_t lm_i2pair(uint32_t d) {
-  const uint32_t e = (d & 0x00030003u) ^ 0x64026402u;
-  const h2v r = __builtin_bit_cast(h2v, e) - h2v{(_Float16)1026.0f, (_Float16)1026.0f};
-  return __builtin_bit_cast(uint32_t, r);
+  return lm_ipair<E>(d & 0x00030003u, 2u, 2.0f);
 }
 // Two int1 codes at bits 0 and 16 of d (other bits ignored): code 0 is
 // +1 and code 1 is -1 (the reference's 1-bit grid), so the code is the f16
-// sign bit of 1.0.
-__device__ __forceinline__ uint32_t lm_i1pair(uint32_t d) { return ((d & 0x00010001u) << 15) | 0x3C003C00u; }
+// sign bit of 2^-E.
+template <int E = 0>
+__device__ __forceinline__ uint32_t lm_i1pair(uint32_t d) {
+  return ((d & 0x00010001u) << 15) | ((0x3C00u - ((uint32_t)E << 10)) * 0x00010001u);
+}
 // Weight formats: the code width in the low 4 bits, 16 for float grids
 enum : int { LM_I1 = 1, LM_I2 = 2, LM_I4 = 4, LM_I8 = 8, LM_F4 = 16 + 4, LM_F8 = 16 + 8 };
 __host__ __device__ constexpr int lm_bits(int fmt) { return fmt & 15; }
@@ -58,13 +64,14 @@ inline int lm_format(int kind, int bits) {
   if (kind == MXK_KIND_FLOAT) return bits == 4 ? LM_F4 : bits == 8 ? LM_F8 : 0;
   return 0;
 }
-// Two codes of a format (layout of its width) as an f16 B-operand pair
-template <int FMT>
+// Two codes of a format (layout of its width) as an f16 B-operand pair (integer
+// codes: times 2^-E)
+template <int FMT, int E = 0>
 __device__ __forceinline__ uint32_t lm_pair(uint32_t d) {
-  if constexpr (FMT == LM_I4) return lm_i4pair(d);
-  else if constexpr (FMT == LM_I8) return lm_i8pair(d);
-  else if constexpr (FMT == LM_I2) return lm_i2pair(d);
-  else if constexpr (FMT == LM_I1) return lm_i1pair(d);
+  if constexpr (FMT == LM_I4) return lm_i4pair<E>(d);
+  else if constexpr (FMT == LM_I8) return lm_i8pair<E>(d);
+  else if constexpr (FMT == LM_I2) return lm_i2pair<E>(d);
+  else if constexpr (FMT == LM_I1) return lm_i1pair<E>(d);
   else return fp_code_pair_f16<lm_bits(FMT)>(d);
 }
 
@@ -88,8 +95,8 @@ __host__ __device__ constexpr uint32_t lm_sel_f(int a, int b) {
 // four floats (F32) or two f16 pairs, in c[0] and c[2].  One asm statement: an
 // instruction that writes the high half of a register may not be followed at once
 // by one that reads it, and the compiler, which may move single asm statements
-// about, does not see that they do.  (The two wait states before an MFMA:
-// lm_settle.)
+// about, does not see that they do.  Here another one always lies between, and
+// the last two write low halves.  (The two wait states before an MFMA: lm_settle.)
 template <bool F32>
 __device__ __forceinline__ void lm_split4(const uint32_t (&c)[4], const float (&s)[4], uint32_t& h0, uint32_t& h1,
                                           uint32_t& l0, uint32_t& l1) {
@@ -98,11 +105,10 @@ __device__ __forceinline__ void lm_split4(const uint32_t (&c)[4], const float (&
         "v_fma_mixlo_f16 %1, %6, %10, 0 op_sel_hi:[0,0,0]\n\t"
         "v_fma_mixhi_f16 %0, %5, %9, 0 op_sel_hi:[0,0,0]\n\t"
         "v_fma_mixhi_f16 %1, %7, %11, 0 op_sel_hi:[0,0,0]\n\t"
-        "v_fma_mixlo_f16 %2, %4, %8, -%0 op_sel_hi:[0,0,1]\n\t"
-        "v_fma_mixlo_f16 %3, %6, %10, -%1 op_sel_hi:[0,0,1]\n\t"
         "v_fma_mixhi_f16 %2, %5, %9, -%0 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
         "v_fma_mixhi_f16 %3, %7, %11, -%1 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
-        "s_nop 0"
+        "v_fma_mixlo_f16 %2, %4, %8, -%0 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %3, %6, %10, -%1 op_sel_hi:[0,0,1]"
         : "=&v"(h0), "=&v"(h1), "=&v"(l0), "=&v"(l1)
         : "v"(c[0]), "v"(c[1]), "v"(c[2]), "v"(c[3]), "v"(s[0]), "v"(s[1]), "v"(s[2]), "v"(s[3]));
   } else {
@@ -110,11 +116,10 @@ __device__ __forceinline__ void lm_split4(const uint32_t (&c)[4], const float (&
         "v_fma_mixlo_f16 %1, %5, %8, 0 op_sel_hi:[1,0,0]\n\t"
         "v_fma_mixhi_f16 %0, %4, %7, 0 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\t"
         "v_fma_mixhi_f16 %1, %5, %9, 0 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\t"
-        "v_fma_mixlo_f16 %2, %4, %6, -%0 op_sel_hi:[1,0,1]\n\t"
-        "v_fma_mixlo_f16 %3, %5, %8, -%1 op_sel_hi:[1,0,1]\n\t"
         "v_fma_mixhi_f16 %2, %4, %7, -%0 op_sel:[1,0,1] op_sel_hi:[1,0,1]\n\t"
         "v_fma_mixhi_f16 %3, %5, %9, -%1 op_sel:[1,0,1] op_sel_hi:[1,0,1]\n\t"
-        "s_nop 0"
+        "v_fma_mixlo_f16 %2, %4, %6, -%0 op_sel_hi:[1,0,1]\n\t"
+        "v_fma_mixlo_f16 %3, %5, %8, -%1 op_sel_hi:[1,0,1]"
         : "=&v"(h0), "=&v"(h1), "=&v"(l0), "=&v"(l1)
         : "v"(c[0]), "v"(c[2]), "v"(s[0]), "v"(s[1]), "v"(s[2]), "v"(s[3]));
   }

@@ -37,8 +37,8 @@
 // whatever the input magnitudes; the epilogue multiplies by 2^-(ex + es).
 // Terms far below a row's largest keep an absolute error of at most 2^-25 of
 // the scaled units.  ([N][K] x at [1, 2) lost most of the terms that are of x
-// large where the weight is small; the factor 2^-14 on the block scales: 105.6
-// -> 107.5 us at the size above.)
+// large where the weight is small; the fragments of integer codes hold c 2^-14, at
+// no cost, and the scales of float grids take it.)
 //
 // Work split.  A workgroup of 8 waves owns 128 output columns, BM = 32 WM
 // rows and a range of K in stages of 256 rows.  Per stage the 8 waves decode
@@ -212,7 +212,7 @@ __device__ __forceinline__ void nk_store(const NkCodes<lm_bits(FMT)>& c, uint8_t
         const uint32_t d = __builtin_amdgcn_perm(sh, wd, lm_sel(v, v));
         u4v f;
 #pragma unroll
-        for (int p = 0; p < 4; ++p) f[p] = lm_pair<FMT>(d >> (2 * p));
+        for (int p = 0; p < 4; ++p) f[p] = lm_pair<FMT, LM_X_TOP>(d >> (2 * p));
         *reinterpret_cast<u4v*>(sB + lm_frag_off(2 * q + s, t, j + 16 * v)) = f;
       }
     }
@@ -231,8 +231,8 @@ __device__ __forceinline__ void nk_store(const NkCodes<lm_bits(FMT)>& c, uint8_t
 #pragma unroll
         for (int bb = 0; bb < 2; ++bb) {
           const uint32_t d = __builtin_amdgcn_perm(sh, wd, lm_sel(2 * vl + bb, 2 * vl + bb));
-          f[2 * bb] = lm_pair<FMT>(d);
-          f[2 * bb + 1] = lm_pair<FMT>(d >> 4);
+          f[2 * bb] = lm_pair<FMT, LM_X_TOP>(d);
+          f[2 * bb + 1] = lm_pair<FMT, LM_X_TOP>(d >> 4);
         }
         *reinterpret_cast<u4v*>(sB + lm_frag_off(2 * q + (sv >> 1), t, j + 16 * (2 * (sv & 1) + vl))) = f;
       }
@@ -248,7 +248,7 @@ __device__ __forceinline__ void nk_store(const NkCodes<lm_bits(FMT)>& c, uint8_t
         const uint32_t lo4 = c.w[h][v] & 0x0F0F0F0Fu, hi4 = (c.w[h][v] >> 4) & 0x0F0F0F0Fu;
         u4v f;
 #pragma unroll
-        for (int p = 0; p < 4; ++p) f[p] = lm_pair<FMT>(__builtin_amdgcn_perm(hi4, lo4, lm_sel(p, p)));
+        for (int p = 0; p < 4; ++p) f[p] = lm_pair<FMT, LM_X_TOP>(__builtin_amdgcn_perm(hi4, lo4, lm_sel(p, p)));
         *reinterpret_cast<u4v*>(sB + lm_frag_off(ks, t, j + 16 * v)) = f;
       }
     }
@@ -266,7 +266,7 @@ __device__ __forceinline__ void nk_store(const NkCodes<lm_bits(FMT)>& c, uint8_t
         for (int p = 0; p < 4; ++p) {
           const uint32_t wd = c.w[h][2 * e + (p >> 1)];
           const int b = 2 * (p & 1);
-          f[p] = lm_pair<FMT>(__builtin_amdgcn_perm(wd, wd, lm_sel_f<FMT>(b, b + 1)));
+          f[p] = lm_pair<FMT, LM_X_TOP>(__builtin_amdgcn_perm(wd, wd, lm_sel_f<FMT>(b, b + 1)));
         }
         *reinterpret_cast<u4v*>(sB + lm_frag_off(ks, t, j + 16 * g)) = f;
       }
@@ -304,7 +304,7 @@ __device__ __forceinline__ void nk_store_tiled(const NkCodes<4>& c, uint8_t* sB,
     for (int v = 0; v < 4; ++v) {
       u4v f;
 #pragma unroll
-      for (int p = 0; p < 4; ++p) f[p] = lm_i4pair(c.w[h][2 * (v >> 1) + (p >> 1)] >> (8 * (p & 1) + 4 * (v & 1)));
+      for (int p = 0; p < 4; ++p) f[p] = lm_i4pair<LM_X_TOP>(c.w[h][2 * (v >> 1) + (p >> 1)] >> (8 * (p & 1) + 4 * (v & 1)));
       *reinterpret_cast<u4v*>(sB + lm_frag_off(ks, t, j + 16 * v)) = f;
     }
   }
@@ -436,11 +436,12 @@ __global__ __launch_bounds__(LM_THREADS, 1) void k_linear_mfma(
   };
   // fold the block sums into acc with the block's scale of each column
   // (blocks past K: padding rows, P holds exact zeros and s8 zeros).  x's 2^14
-  // leaves here, so that acc holds no larger values than the product of x at [1, 2)
+  // left with the integer codes (their fragments hold c 2^-14) or leaves here, so
+  // that acc holds no larger values than the product of x at [1, 2)
   auto fold = [&](const float (&s8)[8]) {
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
-      const float s = s8[t] * (1.0f / (1 << LM_X_TOP));
+      const float s = lm_post(FMT) != 1.0f ? s8[t] * (1.0f / (1 << LM_X_TOP)) : s8[t];
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
