@@ -49,7 +49,9 @@
 // such terms 64 k at a time, and a lane sums its 4 rows x 8 columns of a row tile
 // side by side until all are NaN.  64 x 2048 x 1001 int8, 107 us (scalar kernel
 // 368): with a NaN 104 us, with infinities in every third row 571 (each output
-// by one lane over all of K: 3.3 and 52 ms).
+// by one lane over all of K: 3.3 and 52 ms).  Where K is split, the second kernel
+// finds them, one lane per output, and that lane sums all of K: 20 x 16384 x 1001
+// 75 us, with infinities 1.7 ms (scalar kernel 3.9).
 #include "mxk_linear_mfma.h"
 
 #include <algorithm>
