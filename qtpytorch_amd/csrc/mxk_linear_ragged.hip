@@ -514,12 +514,16 @@ __global__ __launch_bounds__(256) void k_linear_ragged_reduce(RgArgs a) {
 }
 
 // Workgroups 0 .. M - 1: a row of x each (lm_prep_row); the others the largest
-// finite |scale|: of four columns each ([N][K], one wave per column), or of the
-// groups of columns of 8 column tiles over one of RG_CHUNKS parts of K each
-// ([K][N]; 8 threads side by side read the scales of 8 tiles, which lie together:
-// with one tile per workgroup every lane met a line of its own, 15 us at 4096 x
-// 50257).  Blocks of 128 and more: at most two meet a row of a tile, and the
-// groups of 32 are kept in registers (groups of 8 in LDS: 7.7 us there).
+// finite |scale|: of four columns each ([N][K], one wave per column), or ([K][N]) of
+// the groups of columns of a run of column tiles over one of RG_CHUNKS parts of K.
+// Blocks of 128 and more: 8 tiles, a row of them by 8 threads side by side, since
+// their scales lie together (one tile per workgroup: 15 us at 4096 x 50257, so 5; few
+// tiles as well: 5.2 at 4096 x 4098, so 4.4); at most two blocks meet a row of a
+// tile, and the groups of 32 are kept in registers.  Smaller blocks: one tile, 16
+// threads to a row, a thread to each group of 8.  Its loads depend on nothing, 16 at a
+// time; a loop over a row's blocks with a maximum in LDS for each waited on every one
+// (16 x 4096 x 1000 int8, blocks of 64: call 37.4 -> 22 us; with 2, 4 tiles per workgroup the pass takes
+// 6.1 and 9.6 us, so 4.4; blocks of 64 at 4096 x 50257 15.2, 18.6, so 14.2).
 template <typename T, bool VEC, bool WT, bool LO>
 __global__ __launch_bounds__(256) void k_linear_ragged_prep(const T* __restrict__ x, RgArgs a, _Float16* __restrict__ xh,
                                                             _Float16* __restrict__ xl, int* __restrict__ ex,
@@ -540,11 +544,12 @@ __global__ __launch_bounds__(256) void k_linear_ragged_prep(const T* __restrict_
     mx = group_max<64>(mx);
     if (lane == 0) smax[n] = mx;
   } else {
-    __shared__ uint32_t gm[128];  // [wave][tile][4 groups of 32], or [tile][16 of 8]
-    const uint32_t tile0 = (uint32_t)(b / RG_CHUNKS) * 8u, tile = tile0 + (tid & 7), ch = (uint32_t)(b % RG_CHUNKS);
+    __shared__ uint32_t gm[128];  // [wave][tile][4 groups of 32], or [16 groups of 8]
+    const uint32_t ch = (uint32_t)(b % RG_CHUNKS);
     const uint32_t N = (uint32_t)a.N, K = (uint32_t)a.K, tiles = (uint32_t)a.tiles, per = (K + RG_CHUNKS - 1) / RG_CHUNKS;
-    const uint32_t k1 = min(K, (ch + 1) * per), n0 = 128u * tile, cl = min(128u, N - n0) - 1u;  // (cl: its last column)
+    const uint32_t k1 = min(K, (ch + 1) * per);
     if (a.gsh == 5) {
+      const uint32_t tile0 = (uint32_t)(b / RG_CHUNKS) * 8u, tile = tile0 + (tid & 7), n0 = 128u * tile, cl = min(128u, N - n0) - 1u;  // (cl: its last column)
       uint32_t m[4] = {0u, 0u, 0u, 0u};
       if (tile < tiles) {
         // the loads of 8 rows at a time (past the last row: that row again)
@@ -577,20 +582,30 @@ __global__ __launch_bounds__(256) void k_linear_ragged_prep(const T* __restrict_
         smax[ch * 4u * tiles + 4u * tile0 + tid] =
             __uint_as_float(max(max(gm[tid], gm[32 + tid]), max(gm[64 + tid], gm[96 + tid])));
     } else {
-      if (tid < 128) gm[tid] = 0u;
-      __syncthreads();
-      if (tile < tiles) {
-        for (uint32_t k = ch * per + (tid >> 3); k < k1; k += 32) {
-          const uint32_t f = k * N + n0;
-          for (uint32_t q = f >> a.sh; q <= (f + cl) >> a.sh; ++q) {
-            const uint32_t c0 = max(q << a.sh, f) - f, c1 = min((q << a.sh) + a.block - 1u - f, cl);
-            const uint32_t v = rg_finite(a.scales[q]);
-            for (uint32_t c = c0 >> 3; c <= c1 >> 3; ++c) atomicMax(&gm[16 * (tid & 7) + c], v);
+      // a thread: one group (at most two blocks meet its 8 columns) in every 16th row
+      const uint32_t tile = (uint32_t)(b / RG_CHUNKS), gi = (uint32_t)tid & 15u, n = 128u * tile + 8u * gi;
+      uint32_t m = 0u;
+      if (n < N) {
+        const uint32_t cl = min(7u, N - 1u - n);
+        for (uint32_t k = ch * per + (tid >> 4); k < k1; k += 128) {
+          float s0[8], s1[8];
+#pragma unroll
+          for (uint32_t u = 0; u < 8; ++u) {
+            const uint32_t f = min(k + 16u * u, k1 - 1u) * N + n;
+            s0[u] = a.scales[f >> a.sh];
+            s1[u] = a.scales[(f + cl) >> a.sh];
           }
+#pragma unroll
+          for (int u = 0; u < 8; ++u) m = max(m, max(rg_finite(s0[u]), rg_finite(s1[u])));
         }
       }
+#pragma unroll
+      for (int o = 16; o < 64; o <<= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o));
+      if (lane < 16) gm[(tid >> 6) * 16 + lane] = m;
       __syncthreads();
-      if (tid < 128 && tile0 + tid / 16 < tiles) smax[ch * 16u * tiles + 16u * tile0 + tid] = __uint_as_float(gm[tid]);
+      if (tid < 16)
+        smax[ch * 16u * tiles + 16u * tile + tid] =
+            __uint_as_float(max(max(gm[tid], gm[16 + tid]), max(gm[32 + tid], gm[48 + tid])));
     }
   }
 }
@@ -673,13 +688,13 @@ void rg_launch_s(const RgPlan& p, const RgArgs& a, bool xlo, bool straddle, hipS
 }
 
 // workgroups of the prepass that find the largest scales
-int64_t rg_max_groups(bool nk, int64_t N) {
-  return nk ? ceil_div(N, 4) : RG_CHUNKS * ceil_div(ceil_div(N, 128), 8);
+int64_t rg_max_groups(bool nk, const RgArgs& a) {
+  return nk ? ceil_div(a.N, 4) : RG_CHUNKS * ceil_div(a.tiles, a.gsh == 5 ? 8 : 1);
 }
 
 template <bool WT, typename T>
 void rg_prep(const RgPlan& p, const RgArgs& a, _Float16* xh, _Float16* xl, int* ex, float* smax, hipStream_t st) {
-  const dim3 grid((unsigned)(a.M + rg_max_groups(WT, a.N)));
+  const dim3 grid((unsigned)(a.M + rg_max_groups(WT, a)));
   const T* x = (const T*)a.x;
   const bool vec = aligned16(x) && (a.K * (int64_t)sizeof(T)) % 16 == 0;
   // only the 64-row tiles have a form without lo

@@ -255,6 +255,30 @@ def test_non_finite_rows_take_no_longer_than_the_scalar_kernel(qa, nt):
     assert max(t[:2]) < 3 * base and t[2] < 8 * fp32
 
 
+def test_small_blocks_take_little_longer(qa):
+    """Few rows, few columns: the largest scales of blocks of 8 to 64 are found about as
+    fast as those of 128 (one load after the other: 1.7 to 2.8 times the call)."""
+    M, K, N = 16, 4096, 1000
+
+    def us(block):
+        x, p, s, _ = _case(M, K, N, "int8d", block, False, torch.float32)
+        x, p, s = x.cuda(), p.cuda(), s.cuda()
+        best = float("inf")
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(20):
+                qa.ops.linear_wq(x, p, s, "int8d", K, N, block)
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b) * 1e3 / 20)
+        return best
+
+    t = {block: us(block) for block in (128, 8, 32, 64)}
+    print(t)
+    assert max(t.values()) < 1.4 * t[128]
+
+
 @pytest.mark.parametrize("nt", [False, True], ids=["kn", "nk"])
 def test_keeps_no_workspace(qa, nt):
     """A call's scratch memory (x again, and the partial sums) goes back with it."""
