@@ -155,7 +155,7 @@ __device__ __forceinline__ uint64_t rg_odd(const RgArgs& a, int64_t mt, uint32_t
   const int64_t kl = min(k0 + lane, a.K - 1);
   bool odd = false, all = false;
   auto rows = [&](const auto* x, uint32_t emask) {
-#pragma unroll
+#pragma unroll 4
     for (int r = 0; r < 16; ++r) {
       const int64_t m = min(mt + r, (int64_t)a.M - 1);
       const uint32_t b = x[m * a.K + kl];
@@ -178,6 +178,59 @@ __device__ __forceinline__ uint64_t rg_odd(const RgArgs& a, int64_t mt, uint32_t
   }
   const uint64_t in = a.K - k0 >= 64 ? ~0ull : (1ull << (a.K - k0)) - 1;
   return (__ballot(all) != 0 ? ~0ull : __ballot(odd)) & in;
+}
+
+// The outputs of the row tile at mt and the column tile at n0 that came out as NaN
+// without one in their row, summed again by the wave that wrote them.  A
+// function of its own, which reads the kernel's arguments (args: where they lie)
+// itself: inlined, what it needs of them stayed in registers across the product's
+// loop and 18 to 34 more of the loop's own spilled (64-row tiles of fp32 x: 48 x
+// 4096 x 1000 int8 37.6 -> 44.6 us).
+template <int FMT, bool WT>
+__device__ __attribute__((noinline)) void rg_rescue(const RgArgs* args, int64_t mt, uint32_t n0, int lane) {
+  const RgArgs& a = *args;
+  const int64_t m = mt + 4 * (lane >> 4);
+  const uint32_t nl = n0 + 8u * (lane & 15);
+  uint32_t todo = 0u;  // bit 8 q + t: the output of row m + q and column nl + t (which this lane wrote)
+  for (int e = 0; e < 32; ++e) {
+    const int64_t mr = m + (e >> 3), n = (int64_t)nl + (e & 7);
+    if (mr >= a.M || n >= a.N || a.ex[mr] == LM_NAN_ROW) continue;
+    const float v = a.out[mr * a.N + n];
+    todo |= (v != v ? 1u : 0u) << e;
+  }
+  if (__ballot(todo != 0u) == 0) return;
+  float y[4][8];
+#pragma unroll
+  for (int e = 0; e < 32; ++e) y[e >> 3][e & 7] = 0.0f;
+  bool open = true;
+#pragma unroll 1
+  for (int64_t k0 = 0; k0 < a.K && open; k0 += 64) {
+    uint64_t odd = rg_odd<WT>(a, mt, n0, k0, lane);
+    while (odd != 0 && open) {
+      const int64_t k = k0 + __builtin_ctzll(odd);
+      odd &= odd - 1;
+      float xv[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) xv[q] = rg_x(a, min(m + q, (int64_t)a.M - 1), k);
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        const int64_t n = min((int64_t)nl + t, a.N - 1);
+        const float w = rg_weight<FMT>(a, (uint32_t)(WT ? n * a.K + k : k * a.N + n));
+#pragma unroll
+        for (int q = 0; q < 4; ++q) y[q][t] = __builtin_fmaf(xv[q], w, y[q][t]);
+        if (t & 1) asm volatile("" ::: "memory");  // (addresses of two columns at a time, not of eight: no stack)
+      }
+      uint32_t nan = 0u;
+#pragma unroll
+      for (int e = 0; e < 32; ++e) nan |= (y[e >> 3][e & 7] != y[e >> 3][e & 7] ? 1u : 0u) << e;
+      open = __ballot((todo & ~nan) != 0u) != 0;
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 32; ++e) {
+    const int64_t n = (int64_t)nl + (e & 7);
+    if ((todo >> e) & 1u) a.out[(m + (e >> 3)) * a.N + n] = y[e >> 3][e & 7] + (a.bias ? a.bias[n] : 0.0f);
+  }
 }
 
 // the finished output from its sum in the scaled units
@@ -450,48 +503,8 @@ __global__ __launch_bounds__(RG_WAVES * 64, 2) void k_linear_ragged(RgArgs a) {
     }
   if (a.part || __ballot(bad) == 0) return;
 #pragma unroll 1
-  for (int i = 0; i < RT; ++i) {
-    const int64_t mt = m0 + 16 * i, m = mt + 4 * g;
-    uint32_t todo = 0u;  // bit 8 q + t: the output of row m + q and column nl + t (which this lane wrote)
-    for (int e = 0; e < 32; ++e) {
-      const int64_t mr = m + (e >> 3), n = (int64_t)nl + (e & 7);
-      if (mr >= a.M || n >= a.N || a.ex[mr] == LM_NAN_ROW) continue;
-      const float v = a.out[mr * a.N + n];
-      todo |= (v != v ? 1u : 0u) << e;
-    }
-    if (__ballot(todo != 0u) == 0) continue;
-    float y[4][8];
-#pragma unroll
-    for (int e = 0; e < 32; ++e) y[e >> 3][e & 7] = 0.0f;
-    bool open = true;
-#pragma unroll 1
-    for (int64_t k0 = 0; k0 < a.K && open; k0 += 64) {
-      uint64_t odd = rg_odd<WT>(a, mt, n0, k0, lane);
-      while (odd != 0 && open) {
-        const int64_t k = k0 + __builtin_ctzll(odd);
-        odd &= odd - 1;
-        float xv[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) xv[q] = rg_x(a, min(m + q, (int64_t)a.M - 1), k);
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-          const int64_t n = min((int64_t)nl + t, a.N - 1);
-          const float w = rg_weight<FMT>(a, (uint32_t)(WT ? n * a.K + k : k * a.N + n));
-#pragma unroll
-          for (int q = 0; q < 4; ++q) y[q][t] = __builtin_fmaf(xv[q], w, y[q][t]);
-        }
-        uint32_t nan = 0u;
-#pragma unroll
-        for (int e = 0; e < 32; ++e) nan |= (y[e >> 3][e & 7] != y[e >> 3][e & 7] ? 1u : 0u) << e;
-        open = __ballot((todo & ~nan) != 0u) != 0;
-      }
-    }
-#pragma unroll
-    for (int e = 0; e < 32; ++e) {
-      const int64_t n = (int64_t)nl + (e & 7);
-      if ((todo >> e) & 1u) a.out[(m + (e >> 3)) * a.N + n] = y[e >> 3][e & 7] + (a.bias ? a.bias[n] : 0.0f);
-    }
-  }
+  for (int i = 0; i < RT; ++i)
+    rg_rescue<FMT, WT>((const RgArgs*)__builtin_amdgcn_kernarg_segment_ptr(), m0 + 16 * i, n0, lane);
 }
 
 // outputs from the K splits' partials, summed in split order
