@@ -169,7 +169,7 @@ size_t mxk_linear_workspace(int64_t M, int64_t K, int64_t N, int bits, int block
 /* Workspace bytes with which mxk_linear_wq and mxk_linear_wq_nt run the
  * matrix-core kernel for weights that neither of their workspace queries
  * counts: N (mxk_linear_wq) or K (mxk_linear_wq_nt) no multiple of 128, or
- * blocks other than 128 (at least 8), 1-, 2-, 4- and 8-bit codes on 4-byte
+ * blocks other than 128 (at least 8), K at least 32, 1-, 2-, 4- and 8-bit codes on 4-byte
  * aligned buffers of whole 4-byte words.  0 for shapes the kernel does not
  * take.  The workspace is optional: with a smaller one (or none) the scalar
  * kernel runs.  Its first 64 KiB are left alone; the rest need not be

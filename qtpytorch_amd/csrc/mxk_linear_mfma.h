@@ -201,7 +201,8 @@ constexpr int LM_X_TOP = 14;
 constexpr int LM_NAN_ROW = 1 << 20;
 
 // Row m of x: ex[m] such that its largest |x| times 2^ex lies in [2^TOP,
-// 2^(TOP + 1)) (0 for a zero row), and x * 2^ex zero-padded to Kp columns, as
+// 2^(TOP + 1)) (0 for a zero row), and x * 2^ex on Kp columns, those from Kz on
+// moved to the end and zeros before them (Kz = K: zeros at the end), as
 // fp32 (SPLIT false) or as f16 hi + lo (SPLIT true: hi = RN16(v), lo = RN16(v -
 // hi), v - hi exact in fp32; a value keeps 2^-25, so 2^(-25 - TOP) of its row's
 // largest).  VEC: 16-byte rows (K * sizeof(T) % 16 == 0, x
@@ -233,7 +234,7 @@ __device__ __forceinline__ int64_t lm_prep_m(int64_t b, int64_t M) {
 
 // Row m by one workgroup of 256 threads (red: 4 floats of LDS)
 template <typename T, bool SPLIT, int TOP, bool VEC, bool LO = true>
-__device__ __forceinline__ void lm_prep_row(const T* __restrict__ x, int64_t m, int64_t K, int64_t Kp,
+__device__ __forceinline__ void lm_prep_row(const T* __restrict__ x, int64_t m, int64_t K, int64_t Kp, int64_t Kz,
                                             float* __restrict__ xs, _Float16* __restrict__ xh,
                                             _Float16* __restrict__ xl, int* __restrict__ ex, float* red) {
   static_assert(LO || (SPLIT && sizeof(T) == 2), "fp32 x needs lo");
@@ -281,7 +282,8 @@ __device__ __forceinline__ void lm_prep_row(const T* __restrict__ x, int64_t m, 
       elems(c[q], v);
 #pragma unroll
       for (int u = 0; u < E; ++u) v[u] = __builtin_ldexpf(v[u], e);
-      const int64_t at = lm_xoff(m, ch * E, Kp);  // E <= 8 values within one 8-column group
+      // E <= 8 values within one 8-column group (Kp - K is a multiple of E, as K and Kp are)
+      const int64_t at = lm_xoff(m, ch * E + (ch * E >= Kz ? Kp - K : 0), Kp);
       if constexpr (SPLIT) {
         _Float16 h[E], l[E];
 #pragma unroll
@@ -301,10 +303,13 @@ __device__ __forceinline__ void lm_prep_row(const T* __restrict__ x, int64_t m, 
         for (int u = 0; u < E; u += 4) *reinterpret_cast<f4v*>(xs + at + u) = f4v{v[u], v[u + 1], v[u + 2], v[u + 3]};
       }
     }
-    for (int64_t k = K + tid; k < Kp; k += 256) lm_put<T, SPLIT, LO>(xs, xh, xl, lm_xoff(m, k, Kp), 0.0f);
+    for (int64_t k = Kz + tid; k < Kz + Kp - K; k += 256) lm_put<T, SPLIT, LO>(xs, xh, xl, lm_xoff(m, k, Kp), 0.0f);
   } else {
-    for (int64_t k = tid; k < Kp; k += 256)
-      lm_put<T, SPLIT, LO>(xs, xh, xl, lm_xoff(m, k, Kp), k < K ? __builtin_ldexpf(ElemT<T>::cvt(row[k]), e) : 0.0f);
+    for (int64_t k = tid; k < Kp; k += 256) {
+      const int64_t from = k < Kz ? k : k - (Kp - K);
+      lm_put<T, SPLIT, LO>(xs, xh, xl, lm_xoff(m, k, Kp),
+                           k < Kz || from >= Kz ? __builtin_ldexpf(ElemT<T>::cvt(row[from]), e) : 0.0f);
+    }
   }
 }
 
@@ -344,7 +349,7 @@ __global__ __launch_bounds__(256) void k_linear_mfma_prep_rows(const T* __restri
     }
     return;
   }
-  lm_prep_row<T, SPLIT, SPLIT ? LM_X_TOP : 0, VEC, LO>(x, lm_prep_m(blockIdx.x, M), K, Kp, xs, xh, xl, ex, red);
+  lm_prep_row<T, SPLIT, SPLIT ? LM_X_TOP : 0, VEC, LO>(x, lm_prep_m(blockIdx.x, M), K, Kp, K, xs, xh, xl, ex, red);
 }
 
 inline size_t lm_round(size_t v) { return (v + 255) & ~(size_t)255; }

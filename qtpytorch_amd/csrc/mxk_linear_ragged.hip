@@ -47,11 +47,11 @@
 // Any other one is summed again in fp32, over the terms that are not finite, so
 // that infinities come out as the scalar kernel gives them: the wave looks for
 // such terms 64 k at a time, and a lane sums its 4 rows x 8 columns of a row tile
-// side by side until all are NaN.  64 x 2048 x 1001 int8, 107 us (scalar kernel
-// 368): with a NaN 104 us, with infinities in every third row 571 (each output
+// side by side until all are NaN.  64 x 2048 x 1001 int8, 83 us (scalar kernel
+// 368): with a NaN 79 us, with infinities in every third row 555 (each output
 // by one lane over all of K: 3.3 and 52 ms).  Where K is split, the second kernel
 // finds them, one lane per output, and that lane sums all of K: 20 x 16384 x 1001
-// 75 us, with infinities 1.7 ms (scalar kernel 3.9).
+// 74 us, with infinities 1.7 ms (scalar kernel 3.9).
 #include "mxk_linear_mfma.h"
 
 #include <algorithm>
@@ -274,18 +274,25 @@ __global__ __launch_bounds__(RG_WAVES * 64, 2) void k_linear_ragged(RgArgs a) {
   for (int t = 0; t < 8; ++t)
     esv[t] = rg_exponent<FMT, WT>(a, WT ? min((int64_t)nl + t, a.N - 1) : (int64_t)nl);
 
-  // flat index of group i (row 8g + i, or column 8j + i) of a step
+  // Flat index of group 0 of a step (group i: row 8g + i, or column 8j + i).  The
+  // last step takes the last 32 rows of K, x being zero where the step before has
+  // them too (lm_prep_row): past K it would read the next column ([N][K]) or the
+  // padding, whose scales may be past f16's range under this column's exponent or not
+  // finite, and x's zero times infinity is NaN.  (Zeros in place of these scales, in
+  // that step alone, cut the loop in two blocks and spilled: 300 x 2050 x 4098 int8, fp32
+  // x, 144 us, so 82; without either 125.)
   auto flat0 = [&](int step) -> uint32_t {
-    const uint32_t k = 32u * step + 8u * g;
+    const uint32_t k = (uint32_t)min(32 * step, (int)a.K - 32) + 8u * g;
     return WT ? nl * ldw + k : k * ldw + nl;
   };
   // Loads are issued whether or not the step exists (`dead` offsets lie past
   // every buffer and read zeros), so that the wait counts stay exact.
-  auto load_raw = [&](RgRaw<BITS>& r, int step, bool live) {
+  auto load_raw = [&](RgRaw<BITS>& r, int step, bool live, const int i0 = 0, const int i1 = 8) __attribute__((always_inline)) {
     const uint32_t dead = live ? 0u : LM_OOB;
     uint32_t f = flat0(step);
+    f += i0 * ldw;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = i0; i < i1; ++i) {
       const uint32_t off = (BITS == 8 ? f & ~3u : BITS == 4 ? (f >> 3) * 4u : BITS == 2 ? (f >> 4) * 4u : (f >> 5) * 4u) |
                            dead;
       if constexpr (ND == 3) {
@@ -335,10 +342,11 @@ __global__ __launch_bounds__(RG_WAVES * 64, 2) void k_linear_ragged(RgArgs a) {
   struct Step {
     KnCodes<BITS> c;
     float sa[8], sb[8];
-    uint32_t pre[8];  // bit u: code u of the group lies before its block boundary
+    uint32_t pre[2];  // bit 8 (i % 4) + u of word i / 4: code u of group i lies before its block boundary
   };
   auto take = [&](Step& p, const RgRaw<BITS>& r, int step) {
     uint32_t f = flat0(step);
+    if constexpr (STR) p.pre[0] = p.pre[1] = 0u;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const uint32_t sh = BITS == 8 ? (f & 3u) * 8u : BITS == 4 ? (f & 7u) * 4u : BITS == 2 ? (f & 15u) * 2u : f & 31u;
@@ -353,38 +361,21 @@ __global__ __launch_bounds__(RG_WAVES * 64, 2) void k_linear_ragged(RgArgs a) {
       p.sa[i] = __builtin_ldexpf(__uint_as_float(r.s[i][0]), e);
       if constexpr (STR) {
         p.sb[i] = __builtin_ldexpf(__uint_as_float(r.s[i][1]), e);
-        p.pre[i] = (1u << min(a.block - (f & (a.block - 1u)), 8u)) - 1u;
+        p.pre[i >> 2] |= ((1u << min(a.block - (f & (a.block - 1u)), 8u)) - 1u) << (8 * (i & 3));
       }
       f += ldw;
     }
   };
-  // The step that K ends in: places past K hold the next column's ([N][K]) or the
-  // padding's codes, whose scales this column's exponent may take past f16's
-  // range, and x's zero times infinity is NaN.  Their scales become zeros.  A
-  // block that begins before K's end is this column's own.
-  const int kcut = (a.K & 31) != 0 ? a.steps - 1 : -1;
-  auto cut = [&](Step& p) {
-    const int left = (int)(a.K - 32 * (int64_t)kcut) - 8 * g;  // rows of this lane before K's end
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const bool gone = WT ? left <= 0 : i >= left;
-      p.sa[i] = gone ? 0.0f : p.sa[i];
-      if constexpr (STR) {
-        const bool past = gone || (WT && left < 8 && p.pre[i] >= (1u << left) - 1u);
-        p.sb[i] = past ? 0.0f : p.sb[i];
-      }
-    }
-  };
-  auto tiles = [&](const Step& p, const XA& x) {
+  auto tiles = [&](const Step& p, const XA& x, const int t0, const int t1) __attribute__((always_inline)) {
     auto scale = [&](int i, const int u) __attribute__((always_inline)) -> float {  // of code u of group i
       if constexpr (!STR) return p.sa[i];
       // a mask by v_bfe_i32 and v_bfi: a compare and a select through VCC wait on each other
       uint32_t m;
-      asm("v_bfe_i32 %0, %1, %2, 1" : "=v"(m) : "v"(p.pre[i]), "s"(u));
+      asm("v_bfe_i32 %0, %1, %2, 1" : "=v"(m) : "v"(p.pre[i >> 2]), "s"(8 * (i & 3) + u));
       return __uint_as_float((__float_as_uint(p.sa[i]) & m) | (__float_as_uint(p.sb[i]) & ~m));
     };
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
+    for (int t = t0; t < t1; ++t) {
       u4v bh, bl;
       u4v d = {0u, 0u, 0u, 0u};
       if constexpr (!WT && FMT != LM_I8) d = kn_frag<FMT>(p.c, t);
@@ -434,8 +425,12 @@ __global__ __launch_bounds__(RG_WAVES * 64, 2) void k_linear_ragged(RgArgs a) {
   // This wave's steps s0 + wk, + WK, ...: codes DR steps ahead (few rows: the
   // loads in flight bound it), x one or DR steps ahead while the registers
   // allow it (64-row tiles: requested when the last MFMA of the step has read
-  // it).
+  // it).  64-row tiles of [N][K] weights: column tile t needs the codes of group t
+  // alone, so the second half of the next step's waits until the first half of the
+  // tiles is done, which spares the registers to hold them (int8, fp32 x, 48 x 4096 x
+  // 1000 37.3 us, else 39.1; 300 x 2050 x 4098 82, else 103).
   {
+    constexpr bool HALF = WT && RT == 4;
     constexpr int DR = RT == 1 ? 2 : 1, DX = RT < 4 ? 2 : 1, U = DX;
     RgRaw<BITS> r[DR];
     XA x[DX];
@@ -451,11 +446,15 @@ __global__ __launch_bounds__(RG_WAVES * 64, 2) void k_linear_ragged(RgArgs a) {
         const int cur = st + p * WK, nx = cur + DR * WK;  // a step past s1 computes on zeros
         Step sp;
         take(sp, r[p % DR], cur);
-        if (cur == kcut) cut(sp);
-        load_raw(r[p % DR], nx, nx < s1);
+        load_raw(r[p % DR], nx, nx < s1, 0, HALF ? 4 : 8);
         if constexpr (DX == 2 && DR == 1) load_x(x[p ^ 1], nx, nx < s1);
         __builtin_amdgcn_sched_barrier(0);
-        tiles(sp, x[p]);
+        tiles(sp, x[p], 0, 4);
+        if constexpr (HALF) {
+          load_raw(r[p % DR], nx, nx < s1, 4, 8);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        tiles(sp, x[p], 4, 8);
         if constexpr (DX == DR) load_x(x[p], nx, nx < s1);
       }
     }
@@ -544,7 +543,7 @@ __global__ __launch_bounds__(256) void k_linear_ragged_prep(const T* __restrict_
   __shared__ float sm[4];
   const int tid = threadIdx.x, lane = tid & 63;
   if ((int64_t)blockIdx.x < a.M) {
-    lm_prep_row<T, true, LM_X_TOP, VEC, LO>(x, lm_prep_m(blockIdx.x, a.M), a.K, a.Kp, nullptr, xh, xl, ex, sm);
+    lm_prep_row<T, true, LM_X_TOP, VEC, LO>(x, lm_prep_m(blockIdx.x, a.M), a.K, a.Kp, a.Kp - 32, nullptr, xh, xl, ex, sm);
     return;
   }
   const int64_t b = (int64_t)blockIdx.x - a.M;
@@ -630,12 +629,12 @@ struct RgPlan {
   size_t off_ex = 0, off_es = 0, off_x = 0, off_p = 0, bytes = 0;
 };
 
-// Shapes the kernel takes: flat indices (with a step of rows past the end)
-// and every buffer below 2^31, blocks of a power of two from 8 on
+// Shapes the kernel takes: one step of K at least, flat indices and every buffer
+// below 2^31, blocks of a power of two from 8 on
 bool rg_shape_ok(int64_t M, int64_t K, int64_t N, int bits, int64_t block) {
   const int64_t lim = int64_t(1) << 31;
   if (bits != 1 && bits != 2 && bits != 4 && bits != 8) return false;
-  if (M < 1 || K < 1 || N < 1 || block < 8 || (block & (block - 1)) != 0 || block >= lim || K >= lim / 64 || N >= lim / 64) return false;
+  if (M < 1 || K < 32 || N < 1 || block < 8 || (block & (block - 1)) != 0 || block >= lim || K >= lim / 64 || N >= lim / 64) return false;
   if ((K + 64) * (N + 128) >= lim || M >= lim || 64 * (K + 32) * 2 >= lim) return false;
   return 8 * ceil_div(ceil_div(N, 128), 8) * ceil_div(M, 16) * 16 < lim;
 }

@@ -142,6 +142,18 @@ def test_columns_do_not_see_what_lies_past_k(qa, dt, M, nt):
 
 
 @pytest.mark.parametrize("nt", [False, True], ids=["kn", "nk"])
+@pytest.mark.parametrize("M,src", [(3, torch.float32), (20, torch.bfloat16), (70, torch.float32), (70, torch.bfloat16)])
+@pytest.mark.parametrize("dt", FMTS)
+def test_ends_of_k(qa, dt, M, src, nt):
+    """K around whole steps of 32 (the last step takes the last 32 rows of K, and those
+    that the step before has count once), and below one step."""
+    for K in (31, 32, 33, 40, 63, 64, 65, 95, 164):
+        for N, block in ((40, 8), (131, 128)):
+            x, p, s, wd = _case(M, K, N, dt, block, nt, src)
+            _check(_run(qa, x, p, s, dt, K, N, block, nt), x, wd, nt, block=block)
+
+
+@pytest.mark.parametrize("nt", [False, True], ids=["kn", "nk"])
 @pytest.mark.parametrize("M", [3, 70])
 @pytest.mark.parametrize("dt", FMTS)
 def test_column_magnitudes(qa, dt, M, nt):
