@@ -26,8 +26,8 @@
 // What bounds it: few rows, the decode (about 480 VALU per 32 x 128 step of a
 // wave) and the number of column tiles against CUs; many rows, decode and MFMA
 // in equal parts (a wave decodes its weights for 64 rows).  16 x 4096 x 50257
-// int8: 1149 us on the scalar kernel, here 97.7 (the profiler gives the product
-// 99 and the prepass 6 us, each by itself); VALU instructions take 56% of the
+// int8: 1149 us on the scalar kernel, here 96.8 (the profiler gives the product
+// 98 and the prepass 6 us, each by itself); VALU instructions take 55% of the
 // SIMDs' time, 73% where a CU holds two of the 393 tiles, MFMAs 9%.  1.2e-6 off
 // the 64-bit product there, 3.0e-7 here.
 //
@@ -534,8 +534,8 @@ __global__ __launch_bounds__(256) void k_linear_ragged_reduce(RgArgs a) {
 // tile, and the groups of 32 are kept in registers.  Smaller blocks: one tile, 16
 // threads to a row, a thread to each group of 8.  Its loads depend on nothing, 16 at a
 // time; a loop over a row's blocks with a maximum in LDS for each waited on every one
-// (16 x 4096 x 1000 int8, blocks of 64: call 37.4 -> 22 us; with 2, 4 tiles per workgroup the pass takes
-// 6.1 and 9.6 us, so 4.4; blocks of 64 at 4096 x 50257 15.2, 18.6, so 14.2).
+// (16 x 4096 x 1000 int8, blocks of 64: call 37.4 -> 21.5 us; the pass with 2 and 4 tiles
+// per workgroup 6.1 and 9.6 us, so 4.4; at 4096 x 50257 15.2 and 18.6, so 14.2).
 template <typename T, bool VEC, bool WT, bool LO>
 __global__ __launch_bounds__(256) void k_linear_ragged_prep(const T* __restrict__ x, RgArgs a, _Float16* __restrict__ xh,
                                                             _Float16* __restrict__ xl, int* __restrict__ ex,
